@@ -147,8 +147,7 @@ void readback(State& s, double* dres, double* out, int n) {
     for (int i = 0; i < n; i++) out[i] = s.hres[i];
 }
 
-std::vector<PauliTermDev> pauli_terms(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n,
-                                      bool dm) {
+std::vector<PauliTermDev> dm_pauli_terms(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n) {
     std::vector<PauliTermDev> terms(T);
     for (unsigned t = 0; t < T; t++) {
         uint64_t mxy = 0, myz = 0;
@@ -157,7 +156,7 @@ std::vector<PauliTermDev> pauli_terms(const double* coeffs, unsigned T, const un
             unsigned c = paulis[(uint64_t)t * n + q];
             if (c == 1 || c == 2) mxy |= 1ULL << q;
             if (c == 2 || c == 3) myz |= 1ULL << q;
-            if (c == 2) ph *= dm ? cd(0, -1) : cd(0, 1);
+            if (c == 2) ph *= cd(0, -1);
         }
         cd f = coeffs[t] * ph;
         terms[t] = PauliTermDev{mxy, myz, f.real(), f.imag()};
@@ -661,7 +660,7 @@ int fsa_densitymatrix_expecPauliString(fsa_state* h, const double* coeffs, unsig
         check_paulis(allPaulis, numTerms * s.N);
         flush(s);
         if (numTerms == 0) { out[0] = out[1] = 0; return; }
-        auto terms = pauli_terms(coeffs, numTerms, allPaulis, s.N, true);
+        auto terms = dm_pauli_terms(coeffs, numTerms, allPaulis, s.N);
         auto* dt = (const PauliTermDev*)s.ring.push(terms.data(), terms.size() * sizeof(PauliTermDev));
         double* ws = s.workspace(expec_workspace_doubles(s.N, numTerms) + 8);
         if (s.prec == FSA_FP64) launch_dm_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, dt, numTerms, ws + 8, ws);
@@ -751,11 +750,12 @@ int fsa_statevector_expecPauliSum(fsa_state* h, const double* coeffs, unsigned n
         check_paulis(paulis, numTerms * s.N);
         flush(s);
         if (numTerms == 0) { out[0] = out[1] = 0; return; }
-        auto terms = pauli_terms(coeffs, numTerms, paulis, s.N, false);
-        auto* dt = (const PauliTermDev*)s.ring.push(terms.data(), terms.size() * sizeof(PauliTermDev));
-        double* ws = s.workspace(expec_workspace_doubles(s.N, numTerms) + 8);
-        if (s.prec == FSA_FP64) launch_sv_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, dt, numTerms, ws + 8, ws);
-        else launch_sv_expec<float>(s.stream, (const cx<float>*)s.amps, s.N, dt, numTerms, ws + 8, ws);
+        PauliSum hs = pauli_sum(coeffs, numTerms, paulis, s.N);
+        push_pauli_sum(s.ring, hs);
+        const unsigned G = (unsigned)hs.groups.size();
+        double* ws = s.workspace(sv_expec_workspace_doubles(s.N, G) + 8);
+        if (s.prec == FSA_FP64) launch_sv_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, hs.dgroups, hs.dterms, G, ws + 8, ws);
+        else launch_sv_expec<float>(s.stream, (const cx<float>*)s.amps, s.N, hs.dgroups, hs.dterms, G, ws + 8, ws);
         hip_check(hipGetLastError(), "expec kernel");
         readback(s, ws, out, 2);
     });
@@ -772,10 +772,11 @@ int fsa_statevector_applyPauliSum(fsa_state* h, const double* coeffs, unsigned n
         flush(s);
         o.pending.clear();
         hip_check(hipStreamSynchronize(o.stream), "hipStreamSynchronize");
-        auto terms = pauli_terms(coeffs, numTerms, paulis, s.N, false);
-        auto* dt = (const PauliTermDev*)s.ring.push(terms.data(), terms.size() * sizeof(PauliTermDev));
-        if (s.prec == FSA_FP64) launch_apply_pauli_sum<double>(s.stream, (const cx<double>*)s.amps, (cx<double>*)o.amps, s.N, dt, numTerms);
-        else launch_apply_pauli_sum<float>(s.stream, (const cx<float>*)s.amps, (cx<float>*)o.amps, s.N, dt, numTerms);
+        PauliSum hs = pauli_sum(coeffs, numTerms, paulis, s.N);
+        push_pauli_sum(s.ring, hs);
+        const unsigned G = (unsigned)hs.groups.size();
+        if (s.prec == FSA_FP64) launch_apply_pauli_sum<double>(s.stream, (const cx<double>*)s.amps, (cx<double>*)o.amps, s.N, hs.dgroups, hs.dterms, G);
+        else launch_apply_pauli_sum<float>(s.stream, (const cx<float>*)s.amps, (cx<float>*)o.amps, s.N, hs.dgroups, hs.dterms, G);
         hip_check(hipGetLastError(), "apply Pauli sum");
         hip_check(hipStreamSynchronize(s.stream), "hipStreamSynchronize");
     });

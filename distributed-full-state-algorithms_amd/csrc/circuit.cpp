@@ -17,6 +17,51 @@ using namespace fsa;
 
 namespace fsa {
 
+PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n) {
+    struct Term { uint64_t mxy, myz; double c; uint32_t imag; };
+    std::vector<Term> all(T);
+    for (unsigned t = 0; t < T; t++) {
+        Term& v = all[t];
+        v.mxy = v.myz = 0;
+        for (unsigned q = 0; q < n; q++) {
+            const unsigned code = paulis[(uint64_t)t * n + q];
+            if (code == 1 || code == 2) v.mxy |= 1ULL << q;
+            if (code == 2 || code == 3) v.myz |= 1ULL << q;
+        }
+        // i^{#Y}: 1, i, -1, -i
+        const unsigned ny = (unsigned)__builtin_popcountll(v.mxy & v.myz) & 3u;
+        v.imag = ny & 1u;
+        v.c = (ny & 2u) ? -coeffs[t] : coeffs[t];
+    }
+    std::stable_sort(all.begin(), all.end(), [](const Term& a, const Term& b) {
+        return a.mxy != b.mxy ? a.mxy < b.mxy : a.imag < b.imag;
+    });
+    PauliSum h;
+    h.terms.reserve(T);
+    for (unsigned t = 0; t < T; t++) {
+        if (h.groups.empty() || h.groups.back().mxy != all[t].mxy || h.groups.back().imag != all[t].imag)
+            h.groups.push_back(PauliGroupDev{all[t].mxy, t, t, all[t].imag, 0u});
+        h.groups.back().t1 = t + 1;
+        h.terms.push_back(PauliSignDev{all[t].myz, all[t].c});
+    }
+    for (size_t g = 0, first = 0; g < h.groups.size(); g++) {
+        if ((h.groups[g].mxy ^ h.groups[first].mxy) >> PAULI_CHUNK_BITS) first = g;
+        h.groups[first].run++;
+    }
+    return h;
+}
+
+void push_pauli_sum(ParamRing& ring, PauliSum& h) {
+    // one region: groups, then terms (both multiples of 8 bytes)
+    const size_t gb = h.groups.size() * sizeof(PauliGroupDev), tb = h.terms.size() * sizeof(PauliSignDev);
+    std::vector<char> blob(gb + tb);
+    std::memcpy(blob.data(), h.groups.data(), gb);
+    std::memcpy(blob.data() + gb, h.terms.data(), tb);
+    char* d = static_cast<char*>(ring.push(blob.data(), blob.size()));
+    h.dgroups = reinterpret_cast<const PauliGroupDev*>(d);
+    h.dterms = reinterpret_cast<const PauliSignDev*>(d + gb);
+}
+
 HOp inverse(const HOp& op) {
     HOp v = op;
     switch (op.kind) {
@@ -196,24 +241,11 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
     // the end instead of rescaling the states
     if (renorm) launch_norm2<R>(st, (const cx<R>*)phi.s.amps, phi.s.num(), ws, norms + 1);
 
-    std::vector<PauliTermDev> terms(T);
-    for (unsigned t = 0; t < T; t++) {
-        uint64_t mxy = 0, myz = 0;
-        cd ph = 1.0;
-        for (unsigned q = 0; q < n; q++) {
-            unsigned code = paulis[(uint64_t)t * n + q];
-            if (code == 1 || code == 2) mxy |= 1ULL << q;
-            if (code == 2 || code == 3) myz |= 1ULL << q;
-            if (code == 2) ph *= cd(0, 1);
-        }
-        cd f = coeffs[t] * ph;
-        terms[t] = PauliTermDev{mxy, myz, f.real(), f.imag()};
-    }
-    auto* dt = (const PauliTermDev*)phi.s.ring.push(terms.data(), terms.size() * sizeof(PauliTermDev));
+    PauliSum h = pauli_sum(coeffs, T, paulis, n);
+    push_pauli_sum(phi.s.ring, h);
     auto* a_phi = (cx<R>*)phi.s.amps;
     auto* a_lam = (cx<R>*)lam.s.amps;
-    launch_apply_pauli_sum<R>(st, a_phi, a_lam, n, dt, T);
-
+    launch_apply_pauli_sum<R>(st, a_phi, a_lam, n, h.dgroups, h.dterms, (unsigned)h.groups.size());
 
     // Reverse sweep, op by op: for a gadget, <lambda|P_k|phi> and U_k^dag on phi
     // and on lambda in one pass over both states (k_adjoint_step); any other op

@@ -139,6 +139,18 @@ struct Circuit {
     std::shared_ptr<AdjointScratch> adj;
 };
 
+// A Pauli sum on n qubits (paulis[t * n + q], codes 0..3) in the grouped form
+// of launch_sv_expec and launch_apply_pauli_sum, groups in ascending X/Y mask
+// order and terms in the caller's order within a group.
+struct PauliSum {
+    std::vector<PauliGroupDev> groups;
+    std::vector<PauliSignDev> terms;
+    const PauliGroupDev* dgroups = nullptr;   // set by push_pauli_sum
+    const PauliSignDev* dterms = nullptr;
+};
+PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n);
+void push_pauli_sum(ParamRing& ring, PauliSum& h);
+
 // run ops on the state's stream; eager: each op as its own pass(es)
 void execute(State& s, const std::vector<HOp>& ops, const std::vector<Stage>& stages);
 inline void execute(State& s, const Plan& p) { execute(s, p.ops, p.stages); }

@@ -128,6 +128,15 @@ void launch_inner(hipStream_t s, const cx<R>* a, const cx<R>* b, uint64_t num, d
 // sum over terms of coeff_t * (-i)^{nY_t} * sum_r sign * rho[r + 2^N (r ^ mxy_t)]
 struct PauliTermDev { uint64_t mxy, myz; double fr, fi; };   // factor f = coeff * phase
 uint64_t expec_workspace_doubles(unsigned nbits, unsigned numTerms);
+// A Pauli sum on a statevector, its terms grouped by X/Y mask and by whether
+// coeff * i^{#Y} is real or imaginary: group terms t0 .. t1-1 contribute
+// (1 or i) * sum_t c_t (-1)^{par(k & myz_t)} psi_k to amplitude k ^ mxy
+// run: at the first of consecutive groups that agree in the X/Y bits above the
+// lowest PAULI_CHUNK_BITS ones, how many they are (0 at the others)
+struct PauliGroupDev { uint64_t mxy; uint32_t t0, t1; uint32_t imag, run; };
+constexpr unsigned PAULI_CHUNK_BITS = 11;
+struct PauliSignDev { uint64_t myz; double c; };
+uint64_t sv_expec_workspace_doubles(unsigned n, unsigned numGroups);
 // one adjoint reverse step for a parametrised gadget (kernels_reduce.hip)
 struct AdjointStepDev {
     uint64_t mxy, myz;            // Pauli masks (phase gadget: mxy = 0, myz = its parity mask)
@@ -185,17 +194,14 @@ template <typename R>
 unsigned launch_adjoint_diag(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const AdjointDiagDev& st,
                              double* rows, uint64_t stride);
 template <typename R>
-void launch_pauli_element(hipStream_t s, const cx<R>* a, const cx<R>* b, uint64_t num, PauliTermDev term,
-                          double* ws, double* dout);
-template <typename R>
 void launch_dm_expec(hipStream_t s, const cx<R>* rho, unsigned N, const PauliTermDev* dterms,
                      unsigned numTerms, double* ws, double* dout);
 template <typename R>
-void launch_sv_expec(hipStream_t s, const cx<R>* psi, unsigned n, const PauliTermDev* dterms,
-                     unsigned numTerms, double* ws, double* dout);
+void launch_sv_expec(hipStream_t s, const cx<R>* psi, unsigned n, const PauliGroupDev* dgroups,
+                     const PauliSignDev* dterms, unsigned numGroups, double* ws, double* dout);
 template <typename R>
-void launch_apply_pauli_sum(hipStream_t s, const cx<R>* in, cx<R>* out, unsigned n,
-                            const PauliTermDev* dterms, unsigned numTerms);
+void launch_apply_pauli_sum(hipStream_t s, const cx<R>* in, cx<R>* out, unsigned n, const PauliGroupDev* dgroups,
+                            const PauliSignDev* dterms, unsigned numGroups);
 template <typename R>
 void launch_partial_trace(hipStream_t s, const cx<R>* in, cx<R>* out, unsigned N,
                           const unsigned* sortedTargets, unsigned k);
