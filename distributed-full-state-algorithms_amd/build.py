@@ -30,6 +30,12 @@ COMMON = [
     f"-I{PKG.parent / 'include'}",
 ]
 
+# Kernels that interpret op lists with uniform branches over a large register
+# state: structurizing those branches (the default, needed only for divergent
+# ones) copies the state at every merge.
+UNIFORM = ["-mllvm", "-structurizecfg-skip-uniform-regions"]
+PER_FILE = {"kernels_reduce.hip": UNIFORM}
+
 
 def sources():
     return sorted(list(CSRC.glob("*.hip")) + list(CSRC.glob("*.cpp")))
@@ -38,7 +44,7 @@ def sources():
 def _compile(src: Path, verbose: bool) -> Path:
     obj = OUT_DIR / (src.stem + src.suffix.replace(".", "_") + ".o")
     lang = ["-x", "hip"] if src.suffix == ".hip" else []
-    cmd = [HIPCC, *COMMON, *lang, "-c", str(src), "-o", str(obj)]
+    cmd = [HIPCC, *COMMON, *PER_FILE.get(src.name, []), *lang, "-c", str(src), "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -108,9 +108,8 @@ void add(Circuit& c, HOp op) {
     c.maxQubit = std::max(c.maxQubit, mx);
     c.ops.push_back(std::move(op));
     c.cachedPrec = -1;
+    c.revPrec = -1;
 }
-
-void invalidate(Circuit& c) { c.cachedPrec = -1; }
 
 std::vector<cd> mat_of(const double* g, uint64_t dim) {
     need(g != nullptr, FSA_ERR_ARG, "null gate matrix");
@@ -145,6 +144,127 @@ const Plan& plan_for(Circuit& c, unsigned nq, int prec) {
     return c.cached;
 }
 
+
+// ---- passes of the reverse sweep (k_wave_sweep) ------------------------------
+
+// ops with a register-tile form: diagonal gadgets, Pauli strings with one X/Y
+// qubit, one-target matrices (controls and Z factors anywhere)
+bool sweep_form(const HOp& op) {
+    return op.kind == OP_PHASE || op.kind == OP_MAT1 ||
+           (op.kind == OP_PAULI && __builtin_popcountll(op.mxy) <= 1);
+}
+
+template <typename R>
+constexpr unsigned sweep_bits_total() { return SWEEP_LANE_BITS + sweep_reg_bits<R>(); }
+
+// Stages of the reverse sweep on tiles of 2^sweep_bits_total amplitudes.  Ops
+// move past others they commute with (schedule()); a gadget's gradient term
+// <lambda|P|phi> does not change when such an op is undone before or after it.
+template <typename R>
+const std::vector<Stage>& reverse_stages(Circuit& c, unsigned n, int prec) {
+    if (c.revNq != n || c.revPrec != prec) {
+        const size_t L = c.ops.size();
+        std::vector<HOp> rev(L);
+        for (size_t r = 0; r < L; r++) {
+            const HOp& o = c.ops[L - 1 - r];
+            rev[r].kind = o.kind;
+            rev[r].nd = o.nd;
+            rev[r].touch = o.touch;
+            rev[r].tileable = sweep_form(o);
+        }
+        // the low qubits of one 128-byte line are in every tile
+        constexpr unsigned M = sweep_bits_total<R>(), LOW = sizeof(R) == 8 ? 3u : 4u;
+        c.revStages = schedule(rev, n, n <= M ? SchedParams{n, n} : SchedParams{M, LOW});
+        for (Stage& st : c.revStages)
+            for (int& i : st.ops) i = (int)L - 1 - i;
+        c.revNq = n;
+        c.revPrec = prec;
+    }
+    return c.revStages;
+}
+
+// Tile qubits 0-2 go to lane bits 0-2 (whole lines per access); of the others
+// the G that most ops mix go to register bits, where mixing costs no exchange.
+template <typename R>
+SweepGeom sweep_geom(const Circuit& c, const Stage& st) {
+    constexpr unsigned G = sweep_reg_bits<R>();
+    SweepGeom g;
+    std::memset(&g, 0, sizeof(g));
+    unsigned mixes[64] = {0};
+    for (int oi : st.ops)
+        for (uint64_t m = c.ops[oi].nd; m; m &= m - 1) mixes[__builtin_ctzll(m)]++;
+    std::vector<unsigned> rest(st.tq.begin() + 3, st.tq.end());
+    std::stable_sort(rest.begin(), rest.end(),
+                     [&](unsigned a, unsigned b) { return mixes[a] != mixes[b] ? mixes[a] > mixes[b] : a > b; });
+    std::vector<unsigned> reg(rest.begin(), rest.begin() + G), lane(rest.begin() + G, rest.end());
+    std::sort(reg.begin(), reg.end());
+    std::sort(lane.begin(), lane.end());
+    for (unsigned b = 0; b < 3; b++) g.lane[b] = (uint8_t)st.tq[b];
+    for (unsigned b = 3; b < SWEEP_LANE_BITS; b++) g.lane[b] = (uint8_t)lane[b - 3];
+    for (unsigned b = 0; b < G; b++) g.reg[b] = (uint8_t)reg[b];
+    for (unsigned q : st.tq) g.tileMask |= 1ULL << q;
+    return g;
+}
+
+// the op that undoes `op` on a tile of this geometry
+template <typename R>
+SweepOp sweep_op(const HOp& op, const SweepGeom& geo) {
+    constexpr unsigned G = sweep_reg_bits<R>();
+    SweepOp t;
+    std::memset(&t, 0, sizeof(t));
+    int lb[64], rb[64];
+    for (int q = 0; q < 64; q++) lb[q] = rb[q] = -1;
+    for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) lb[geo.lane[b]] = (int)b;
+    for (unsigned b = 0; b < G; b++) rb[geo.reg[b]] = (int)b;
+    uint32_t rmask = 0;
+    auto split = [&](uint64_t m) {
+        for (; m; m &= m - 1) {
+            const int q = __builtin_ctzll(m);
+            if (lb[q] >= 0) t.lz |= 1u << lb[q];
+            else if (rb[q] >= 0) rmask |= 1u << rb[q];
+            else t.oz |= 1ULL << q;
+        }
+    };
+    if (op.kind == OP_MAT1) {
+        split(op.ctrl);
+        for (uint32_t i = 0; i < (1u << G); i++) if ((i & rmask) == rmask) t.sw |= 1u << i;
+        const unsigned q = op.q[0];
+        t.code = rb[q] >= 0 ? SWEEP_MAT_REG + (uint32_t)rb[q] : (uint32_t)SWEEP_MAT_LANE;
+        t.bit = rb[q] >= 0 ? 0u : (uint32_t)lb[q];
+        for (unsigned i = 0; i < 4; i++) {       // conjugate transpose
+            const cd v = std::conj(op.mat[(i & 1) * 2 + (i >> 1)]);
+            t.f[2 * i] = v.real();
+            t.f[2 * i + 1] = v.imag();
+        }
+        return t;
+    }
+    // a Pauli tensor P is exp(i pi/2 P) up to a phase common to phi and lambda,
+    // which no gradient term sees
+    const bool tensor = op.kind == OP_PAULI && !op.gadget;
+    const double cs = tensor ? 0.0 : std::cos(op.theta), sn = tensor ? 1.0 : std::sin(op.theta);
+    split(op.kind == OP_PHASE ? op.pmask : op.myz);
+    for (uint32_t i = 0; i < (1u << G); i++) if (par32(i & rmask)) t.sw |= 1u << i;
+    const uint32_t ss = t.sw != 0;
+    t.c = cs;
+    if (op.kind == OP_PHASE || op.mxy == 0) {
+        t.code = SWEEP_DIAG + ss;
+        t.g = -sn;                               // exp(-i theta Z..Z)
+        return t;
+    }
+    // exp(-i theta P) = cos - i sin i^{#Y} (...): imaginary factor for X, real for Y (#Y = 1)
+    const unsigned q = (unsigned)__builtin_ctzll(op.mxy);
+    const bool y = (op.mxy & op.myz) != 0;
+    t.g = y ? sn : -sn;
+    if (rb[q] >= 0) {
+        t.code = SWEEP_REG + 4u * (uint32_t)rb[q];
+    } else {
+        t.code = SWEEP_LANE;
+        t.bit = (uint32_t)lb[q];
+        if (y) t.lz |= SWEEP_CONST_SIGN;         // the factor is the partner lane's
+    }
+    t.code += (y ? 0u : 2u) + ss;
+    return t;
+}
 
 // a statevector work state on a stream it does not own
 struct Scratch {
@@ -290,6 +410,76 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
         }
         return d.count;
     };
+    // one op on its own: a gadget by k_adjoint_step, any other by its own kernel
+    auto undo = [&](const HOp& op) {
+        const HOp inv = inverse(op);
+        if (op.param >= 0) {
+            AdjointStepDev d;
+            std::memset(&d, 0, sizeof(d));
+            if (op.kind == OP_PAULI) {
+                d.mxy = op.mxy; d.myz = op.myz;
+                d.fr = op.pw.real(); d.fi = op.pw.imag();
+                d.thr = inv.th.real(); d.thi = inv.th.imag();
+                d.fer = inv.fe.real(); d.fei = inv.fe.imag();
+            } else {
+                d.mxy = 0; d.myz = op.pmask;
+                d.fr = 1.0; d.fi = 0.0;
+                d.phase = 1;
+                d.e0r = std::cos(inv.theta); d.e0i = std::sin(inv.theta);
+                d.e1r = std::cos(inv.theta); d.e1i = -std::sin(inv.theta);
+            }
+            d.slot = (uint32_t)op.param;
+            ProfScope prof("adjoint_step", st);
+            nbs[op.param] = launch_adjoint_step<R>(st, a_phi, a_lam, n, d, rows, stride);
+            hip_check(hipGetLastError(), "adjoint step launch");
+            return;
+        }
+        std::vector<HOp> invs{inv};
+        execute_now(phi.s, invs);
+        execute_now(lam.s, invs);
+    };
+    if (n >= sweep_min_qubits<R>()) {
+        // register-tile passes; stages of one op and ops without such a form alone
+        const std::vector<Stage>& stages = reverse_stages<R>(c, n, psi0.prec);
+        struct Pass { SweepGeom geom; size_t first; unsigned count, grads; };
+        std::vector<SweepOp> sops;
+        std::vector<std::vector<Pass>> passes(stages.size());
+        for (size_t si = 0; si < stages.size(); si++) {
+            if (!stages[si].tiled) continue;
+            const SweepGeom geom = sweep_geom<R>(c, stages[si]);
+            for (int oi : stages[si].ops) {
+                const HOp& op = c.ops[oi];
+                auto& ps = passes[si];
+                if (ps.empty() || (op.param >= 0 && ps.back().grads == SWEEP_MAX_GRADS))
+                    ps.push_back(Pass{geom, sops.size(), 0, 0});
+                SweepOp t = sweep_op<R>(op, geom);
+                if (op.param >= 0) {
+                    const unsigned k = ps.back().grads++;
+                    t.acc = k & 1u ? SWEEP_ACC_SECOND : SWEEP_ACC_FIRST;
+                    t.row = k / 2;
+                    t.slot = (uint32_t)op.param;
+                }
+                ps.back().count++;
+                sops.push_back(t);
+            }
+        }
+        ParamRing::Hold hold(phi.s.ring);        // undo() may push parameters of its own
+        const SweepOp* dops = sops.empty() ? nullptr
+            : static_cast<const SweepOp*>(phi.s.ring.push(sops.data(), sops.size() * sizeof(SweepOp)));
+        for (size_t si = 0; si < stages.size(); si++) {
+            if (!stages[si].tiled) {
+                for (int oi : stages[si].ops) undo(c.ops[oi]);
+                continue;
+            }
+            for (const Pass& p : passes[si]) {
+                ProfScope prof("adjoint_sweep", st);
+                const unsigned nb = launch_sweep<R>(st, a_phi, a_lam, n, p.geom, dops + p.first, p.count, p.grads, rows, stride);
+                hip_check(hipGetLastError(), "adjoint sweep launch");
+                for (size_t i = p.first; i < p.first + p.count; i++)
+                    if (sops[i].acc != SWEEP_ACC_NONE) nbs[sops[i].slot] = nb;
+            }
+        }
+    } else {
     for (size_t k = c.ops.size(); k-- > 0;) {
         const HOp& op = c.ops[k];
         if (qubit_gadget(op) && k > 0 && qubit_gadget(c.ops[k - 1]) && c.ops[k - 1].mxy != op.mxy) {
@@ -335,31 +525,8 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
             k -= d.count - 1;       // the loop's k-- moves past the run
             continue;
         }
-        const HOp inv = inverse(op);
-        if (op.param >= 0) {
-            AdjointStepDev d;
-            std::memset(&d, 0, sizeof(d));
-            if (op.kind == OP_PAULI) {
-                d.mxy = op.mxy; d.myz = op.myz;
-                d.fr = op.pw.real(); d.fi = op.pw.imag();
-                d.thr = inv.th.real(); d.thi = inv.th.imag();
-                d.fer = inv.fe.real(); d.fei = inv.fe.imag();
-            } else {
-                d.mxy = 0; d.myz = op.pmask;
-                d.fr = 1.0; d.fi = 0.0;
-                d.phase = 1;
-                d.e0r = std::cos(inv.theta); d.e0i = std::sin(inv.theta);
-                d.e1r = std::cos(inv.theta); d.e1i = -std::sin(inv.theta);
-            }
-            d.slot = (uint32_t)op.param;
-            ProfScope prof("adjoint_step", st);
-            nbs[op.param] = launch_adjoint_step<R>(st, a_phi, a_lam, n, d, rows, stride);
-            hip_check(hipGetLastError(), "adjoint step launch");
-            continue;
-        }
-        std::vector<HOp> invs{inv};
-        execute_now(phi.s, invs);
-        execute_now(lam.s, invs);
+        undo(op);
+    }
     }
     if (P) {
         auto* dnb = (const uint32_t*)phi.s.ring.push(nbs.data(), nbs.size() * sizeof(uint32_t));

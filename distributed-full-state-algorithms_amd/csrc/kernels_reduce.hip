@@ -8,6 +8,7 @@
 
 #include <cstring>
 #include "launch.hpp"
+#include "wave_sweep.hpp"
 
 namespace fsa {
 
@@ -440,6 +441,100 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
     }
 }
 
+// Register-tile pass of the reverse sweep (wave_sweep.hpp).  Gradient terms
+// accumulate per thread in LDS, two gadgets to a row: lanes below 32 keep the
+// first gadget's sum of lanes l and l + 32, the others the second's, so one
+// exchange folds both and a row of 256 doubles serves two gadgets.
+// Three workgroups of four waves per CU (VGPRs and LDS): more waves hide more
+// of the loads and of the scalar work between ops.
+// 24 qubits FP64, 20 layers of 23 ZZ and 24 X gadgets: 35 passes of 375 us (210 us
+// of them the bare loads and stores) against 160 run passes of 197 us and 40
+// diagonal passes of 193 us; 23 qubits FP32 33 of 153 us against 160 of 43-57 and 40 of 48.
+// Bound by the exchanges between lanes and the FP64 arithmetic.
+template <typename R, int G>
+__global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
+                                                         uint64_t numTiles, SweepGeom geom,
+                                                         const SweepOp* __restrict__ ops, unsigned numOps,
+                                                         unsigned numGrads, double* __restrict__ rows, uint64_t stride) {
+    constexpr int S = 1 << G;
+    __shared__ double acc[SWEEP_MAX_GRADS / 2][BLOCK];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const bool upper = lane >= 32u;
+    for (unsigned k = 0; k < (numGrads + 1) / 2; k++) acc[k][tid] = 0;
+    // The offset of this lane's amplitudes, computed anew for the loads and the
+    // stores of a tile: the empty register constraint hides that the two agree,
+    // or the compiler would keep all of a tile's addresses alive through its ops.
+    auto lane_offset = [&]() {
+        float bits = __builtin_bit_cast(float, lane);
+        asm volatile("" : "+v"(bits));
+        const uint32_t l = __builtin_bit_cast(uint32_t, bits);
+        uint64_t off = 0;
+#pragma unroll
+        for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) off |= (uint64_t)((l >> b) & 1u) << geom.lane[b];
+        return off;
+    };
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint64_t first = adjoint_block<R>() * (BLOCK / 64) + wave, step = (uint64_t)gridDim.x * (BLOCK / 64);
+    auto at = [&](uint64_t base, int i) {
+#pragma unroll
+        for (int b = 0; b < G; b++) if ((i >> b) & 1) base |= 1ULL << geom.reg[b];
+        return base;
+    };
+    for (uint64_t t = first; t < numTiles; t += step) {
+        const uint64_t base = ins0_mask(t, geom.tileMask), in = lane_offset();
+        sweep::Tile<R, S> v;
+#pragma unroll
+        for (int i = 0; i < S; i++) {
+            const cx<R> p = adj_ld<R, true>(phi + at(base, i) + in), l = adj_ld<R, true>(lam + at(base, i) + in);
+            v.px[i] = p.x; v.py[i] = p.y; v.lx[i] = l.x; v.ly[i] = l.y;
+        }
+        auto header = [&](unsigned o) {
+            SweepOp h;
+            h.code = ops[o].code; h.lz = ops[o].lz; h.sw = ops[o].sw; h.acc = ops[o].acc;
+            h.oz = ops[o].oz; h.c = ops[o].c; h.g = ops[o].g;
+            return h;
+        };
+        SweepOp hdr = header(0);
+        double held = 0;                                    // the first gadget's term of the current row
+        for (unsigned o = 0; o < numOps; o++) {
+            const SweepOp next = header(o + 1 < numOps ? o + 1 : o);     // loads while this op runs
+            const double w = sweep::apply<R, G, true>(v, hdr, ops + o, lane, base);
+            if (hdr.acc == SWEEP_ACC_FIRST) {
+                held = w;
+            } else if (hdr.acc == SWEEP_ACC_SECOND) {
+                const double other = __shfl_xor(upper ? held : w, 32, 64);
+                acc[ops[o].row][tid] += (upper ? w : held) + other;
+            }
+            hdr = next;
+        }
+        if (numGrads & 1u) {                                // a last gadget on its own
+            const double other = __shfl_xor(upper ? held : 0.0, 32, 64);
+            acc[numGrads / 2][tid] += (upper ? 0.0 : held) + other;
+        }
+        const uint64_t out = lane_offset();
+#pragma unroll
+        for (int i = 0; i < S; i++) {
+            adj_st<R, true>(phi + at(base, i) + out, mk<R>(v.px[i], v.py[i]));
+            adj_st<R, true>(lam + at(base, i) + out, mk<R>(v.lx[i], v.ly[i]));
+        }
+    }
+    // workgroup sums: gadget 2 k in the lower, 2 k + 1 in the upper lanes of row k
+    unsigned k = 0;
+    for (unsigned o = 0; o < numOps; o++) {
+        if (ops[o].acc == SWEEP_ACC_NONE) continue;
+        const double a = acc[k / 2][tid];
+        double im = upper == ((k & 1u) != 0) ? a : 0.0, dummy = 0;
+        block_sum2(im, dummy);
+        if (tid == 0) {
+            double* row = rows + stride * ops[o].slot + 2 * blockIdx.x;
+            row[0] = 0;
+            row[1] = im;
+        }
+        __syncthreads();    // block_sum2's wave partials are reused by the next gadget
+        k++;
+    }
+}
+
 // A Pauli sum H on a statevector, grouped by X/Y mask (PauliGroupDev): either
 // <psi|H|psi> (EXPEC, one partial per workgroup) or out = H psi.  A thread owns
 // ITEMS amplitudes j = chunk base + 256 i + tid and walks the groups: it takes
@@ -751,6 +846,21 @@ unsigned launch_adjoint_qrun(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq,
     return nb;
 }
 
+// three workgroups per CU, each wave on every (12 * CUs)-th tile; never more than
+// red_blocks(2^nq) rows (a workgroup's four tiles hold 2^11 amplitudes or more)
+template <typename R>
+unsigned launch_sweep(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom, const SweepOp* dops,
+                      unsigned numOps, unsigned numGrads, double* rows, uint64_t stride) {
+    constexpr unsigned G = sweep_reg_bits<R>(), M = SWEEP_LANE_BITS + G;
+    if (nq < M || numOps == 0 || numGrads > SWEEP_MAX_GRADS || (unsigned)__builtin_popcountll(geom.tileMask) != M)
+        fail(FSA_ERR_INTERNAL, "register-tile pass of unsupported shape");
+    const uint64_t numTiles = 1ULL << (nq - M);
+    const unsigned nb = (unsigned)std::min<uint64_t>((numTiles + BLOCK / 64 - 1) / (BLOCK / 64), 768);
+    hipLaunchKernelGGL((k_wave_sweep<R, (int)G>), dim3(nb), dim3(BLOCK), 0, s, phi, lam, numTiles, geom, dops, numOps,
+                       numGrads, rows, stride);
+    return nb;
+}
+
 // ws must hold 2 * numTerms * ceil(2^nbits / EXP_CHUNK) doubles
 template <typename R>
 void launch_dm_expec(hipStream_t s, const cx<R>* rho, unsigned N, const PauliTermDev* dterms,
@@ -863,6 +973,8 @@ void launch_f32_to_f64(hipStream_t s, const cx<float>* in, cx<double>* out, uint
     template void launch_inner<R>(hipStream_t, const cx<R>*, const cx<R>*, uint64_t, double*, double*);       \
     template unsigned launch_adjoint_step<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointStepDev&,       \
                                              double*, uint64_t);                                                \
+    template unsigned launch_sweep<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const SweepGeom&, const SweepOp*,    \
+                                      unsigned, unsigned, double*, uint64_t);                                   \
     template unsigned launch_adjoint_diag<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointDiagDev&,       \
                                              double*, uint64_t);                                                \
     template unsigned launch_adjoint_qrun<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointQubitRunDev&,   \

@@ -108,6 +108,50 @@ template <typename R> constexpr int tile_bits_limit() { return sizeof(R) == 8 ? 
 // register-sweep width: 2^W amplitudes per thread = full tile / 512 threads
 template <typename R> constexpr int sweep_bits() { return sizeof(R) == 8 ? 2 : 4; }
 
+// ---- register-tile sweeps (wave_sweep.hpp) --------------------------------------
+// One op of a pass.  Qubits are lane bits (0..5), register bits (0..G-1) or
+// outside the tile; lz / oz are the lane and outside parts of its Z mask
+// (matrices: control mask), sw has bit i set where slot i's parity is odd
+// (matrices: where slot i's controls are set).  Bit 6 of lz is a constant sign.
+enum SweepCode : uint32_t {       // imag and ss (sw != 0) select the form: + 2 imag + ss
+    SWEEP_DIAG = 0,      // v' = v (c + i g s), s = +-1 by parity (imag always 0 here)
+    SWEEP_LANE = 4,      // Pauli string with its X/Y qubit on lane bit `bit`:
+    SWEEP_REG = 8,       // ... on register bit B (+ 4 B): v' = c v + (imag ? i g : g) s w, w the partner
+    SWEEP_MAT_LANE = 28, // 2x2 matrix f (row-major) on lane bit `bit`
+    SWEEP_MAT_REG = 29,  // ... on register bit B (+ B)
+};
+constexpr uint32_t SWEEP_CONST_SIGN = 64;
+// Gradient terms: of a pass's gadgets, the ones numbered 2 k and 2 k + 1 share
+// accumulator row k (see k_wave_sweep)
+enum SweepAcc : uint32_t { SWEEP_ACC_NONE = 0, SWEEP_ACC_FIRST = 1, SWEEP_ACC_SECOND = 2 };
+struct SweepOp {
+    uint32_t code, lz, sw, acc;
+    uint64_t oz;
+    double c, g;
+    uint32_t bit;
+    uint32_t row;        // accumulator row (SECOND)
+    uint32_t slot;       // row slot of its gradient term
+    uint32_t pad;
+    double f[8];
+};
+constexpr unsigned SWEEP_LANE_BITS = 6;
+// register bits: 64 VGPRs of amplitudes for phi and lambda
+template <typename R> constexpr unsigned sweep_reg_bits() { return sizeof(R) == 8 ? 3u : 4u; }
+// Smallest states that the passes take.  Smaller ones give a pass one to four
+// waves, which run its ops one after another, and the run kernels' launches of
+// a few us each are no slower: 20 layers of ZZ and X gadgets take 1.21 ms either way at 10
+// qubits FP64, and in FP32 1.33 against 1.20 ms at 10, 1.68 against 1.70 at 12.
+template <typename R> constexpr unsigned sweep_min_qubits() { return sizeof(R) == 8 ? 10u : 12u; }
+constexpr unsigned SWEEP_MAX_GRADS = 46;     // gradient terms of a pass: two per 2 KiB row of LDS
+struct SweepGeom {
+    uint64_t tileMask;
+    uint8_t lane[8], reg[8];                 // qubits of the lane and register bits
+};
+// one pass over phi and lambda; returns the number of workgroups (rows per slot)
+template <typename R>
+unsigned launch_sweep(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom, const SweepOp* dops,
+                      unsigned numOps, unsigned numGrads, double* rows, uint64_t stride);
+
 // ---- init / copy / conversion ------------------------------------------------
 template <typename R>
 void launch_init_gaussian(hipStream_t s, cx<R>* a, unsigned nq, uint64_t seed);
