@@ -108,7 +108,7 @@ void add(Circuit& c, HOp op) {
     c.maxQubit = std::max(c.maxQubit, mx);
     c.ops.push_back(std::move(op));
     c.cachedPrec = -1;
-    c.revPrec = -1;
+    c.sweepPrec[0] = c.sweepPrec[1] = -1;
 }
 
 std::vector<cd> mat_of(const double* g, uint64_t dim) {
@@ -145,7 +145,7 @@ const Plan& plan_for(Circuit& c, unsigned nq, int prec) {
 }
 
 
-// ---- passes of the reverse sweep (k_wave_sweep) ------------------------------
+// ---- register-tile passes of the adjoint (k_wave_sweep) -----------------------
 
 // ops with a register-tile form: diagonal gadgets, Pauli strings with one X/Y
 // qubit, one-target matrices (controls and Z factors anywhere)
@@ -153,117 +153,236 @@ bool sweep_form(const HOp& op) {
     return op.kind == OP_PHASE || op.kind == OP_MAT1 ||
            (op.kind == OP_PAULI && __builtin_popcountll(op.mxy) <= 1);
 }
+// the qubit such an op mixes, or -1
+int sweep_mixes(const HOp& op) { return op.nd ? __builtin_ctzll(op.nd) : -1; }
 
-template <typename R>
-constexpr unsigned sweep_bits_total() { return SWEEP_LANE_BITS + sweep_reg_bits<R>(); }
-
-// Stages of the reverse sweep on tiles of 2^sweep_bits_total amplitudes.  Ops
-// move past others they commute with (schedule()); a gadget's gradient term
+// Stages of the forward or reverse (rev) sweep on register tiles.  Ops move past
+// others they commute with (schedule()); a gadget's gradient term
 // <lambda|P|phi> does not change when such an op is undone before or after it.
 template <typename R>
-const std::vector<Stage>& reverse_stages(Circuit& c, unsigned n, int prec) {
-    if (c.revNq != n || c.revPrec != prec) {
+const std::vector<Stage>& sweep_stages(Circuit& c, unsigned n, int prec, bool rev) {
+    if (c.sweepNq[rev] != n || c.sweepPrec[rev] != prec) {
         const size_t L = c.ops.size();
-        std::vector<HOp> rev(L);
+        std::vector<HOp> order(L);
         for (size_t r = 0; r < L; r++) {
-            const HOp& o = c.ops[L - 1 - r];
-            rev[r].kind = o.kind;
-            rev[r].nd = o.nd;
-            rev[r].touch = o.touch;
-            rev[r].tileable = sweep_form(o);
+            const HOp& o = c.ops[rev ? L - 1 - r : r];
+            order[r].kind = o.kind;
+            order[r].nd = o.nd;
+            order[r].touch = o.touch;
+            order[r].tileable = sweep_form(o);
         }
         // the low qubits of one 128-byte line are in every tile
-        constexpr unsigned M = sweep_bits_total<R>(), LOW = sizeof(R) == 8 ? 3u : 4u;
-        c.revStages = schedule(rev, n, n <= M ? SchedParams{n, n} : SchedParams{M, LOW});
-        for (Stage& st : c.revStages)
-            for (int& i : st.ops) i = (int)L - 1 - i;
-        c.revNq = n;
-        c.revPrec = prec;
+        const unsigned M = SWEEP_LANE_BITS + sweep_reg_bits<R>(rev), low = sizeof(R) == 8 ? 3u : 4u;
+        c.sweepStages[rev] = schedule(order, n, n <= M ? SchedParams{n, n} : SchedParams{M, low});
+        if (rev)
+            for (Stage& st : c.sweepStages[rev])
+                for (int& i : st.ops) i = (int)L - 1 - i;
+        c.sweepNq[rev] = n;
+        c.sweepPrec[rev] = prec;
     }
-    return c.revStages;
+    return c.sweepStages[rev];
 }
 
-// Tile qubits 0-2 go to lane bits 0-2 (whole lines per access); of the others
-// the G that most ops mix go to register bits, where mixing costs no exchange.
-template <typename R>
-SweepGeom sweep_geom(const Circuit& c, const Stage& st) {
-    constexpr unsigned G = sweep_reg_bits<R>();
-    SweepGeom g;
-    std::memset(&g, 0, sizeof(g));
-    unsigned mixes[64] = {0};
-    for (int oi : st.ops)
-        for (uint64_t m = c.ops[oi].nd; m; m &= m - 1) mixes[__builtin_ctzll(m)]++;
-    std::vector<unsigned> rest(st.tq.begin() + 3, st.tq.end());
-    std::stable_sort(rest.begin(), rest.end(),
-                     [&](unsigned a, unsigned b) { return mixes[a] != mixes[b] ? mixes[a] > mixes[b] : a > b; });
-    std::vector<unsigned> reg(rest.begin(), rest.begin() + G), lane(rest.begin() + G, rest.end());
-    std::sort(reg.begin(), reg.end());
-    std::sort(lane.begin(), lane.end());
-    for (unsigned b = 0; b < 3; b++) g.lane[b] = (uint8_t)st.tq[b];
-    for (unsigned b = 3; b < SWEEP_LANE_BITS; b++) g.lane[b] = (uint8_t)lane[b - 3];
-    for (unsigned b = 0; b < G; b++) g.reg[b] = (uint8_t)reg[b];
-    for (unsigned q : st.tq) g.tileMask |= 1ULL << q;
-    return g;
-}
+struct SweepPass {
+    SweepGeom geom;
+    size_t first = 0;        // its ops: sops[first .. first + count)
+    unsigned count = 0, grads = 0;
+};
 
-// the op that undoes `op` on a tile of this geometry
+// Turns a stage into passes: places its qubits on lane and register bits, adds
+// exchanges where an op needs a qubit on a register bit, groups diagonal
+// gadgets.  Tile qubits 0-2 stay on lane bits 0-2 (whole lines per access).
 template <typename R>
-SweepOp sweep_op(const HOp& op, const SweepGeom& geo) {
-    constexpr unsigned G = sweep_reg_bits<R>();
-    SweepOp t;
-    std::memset(&t, 0, sizeof(t));
-    int lb[64], rb[64];
-    for (int q = 0; q < 64; q++) lb[q] = rb[q] = -1;
-    for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) lb[geo.lane[b]] = (int)b;
-    for (unsigned b = 0; b < G; b++) rb[geo.reg[b]] = (int)b;
-    uint32_t rmask = 0;
-    auto split = [&](uint64_t m) {
-        for (; m; m &= m - 1) {
-            const int q = __builtin_ctzll(m);
-            if (lb[q] >= 0) t.lz |= 1u << lb[q];
-            else if (rb[q] >= 0) rmask |= 1u << rb[q];
-            else t.oz |= 1ULL << q;
+class SweepBuilder {
+public:
+    SweepBuilder(const Circuit& c, bool rev, std::vector<SweepOp>& sops)
+        : c_(c), rev_(rev), G_(sweep_reg_bits<R>(rev)), sops_(sops) {}
+
+    std::vector<SweepPass> stage(const Stage& st) {
+        place(st);
+        passes_.clear();
+        open(st);
+        for (size_t i = 0; i < st.ops.size(); i++) {
+            const HOp& op = c_.ops[st.ops[i]];
+            const bool grad = rev_ && op.param >= 0;
+            if (grad && passes_.back().grads == SWEEP_MAX_GRADS) {
+                flush_run();
+                close();
+                open(st);
+            }
+            if (grad) passes_.back().grads++;
+            const int q = sweep_mixes(op);
+            if (q < 0) {
+                run_.push_back(&op);
+                continue;
+            }
+            flush_run();
+            if (lane_[4] == q || lane_[5] == q) {
+                // the register bit whose qubit is mixed again last gives way
+                const unsigned l = lane_[4] == q ? 4 : 5;
+                unsigned B = 0;
+                size_t far = 0;
+                for (unsigned b = 0; b < G_; b++) {
+                    size_t next = i + 1;
+                    while (next < st.ops.size() && sweep_mixes(c_.ops[st.ops[next]]) != reg_[b]) next++;
+                    if (next > far) { far = next; B = b; }
+                }
+                std::swap(lane_[l], reg_[B]);
+                SweepOp t;
+                std::memset(&t, 0, sizeof(t));
+                t.code = SWEEP_SWAP + 5 * (l - 4) + B;
+                emit(t, nullptr);
+            }
+            emit(translate(op), &op);
         }
-    };
-    if (op.kind == OP_MAT1) {
-        split(op.ctrl);
-        for (uint32_t i = 0; i < (1u << G); i++) if ((i & rmask) == rmask) t.sw |= 1u << i;
-        const unsigned q = op.q[0];
-        t.code = rb[q] >= 0 ? SWEEP_MAT_REG + (uint32_t)rb[q] : (uint32_t)SWEEP_MAT_LANE;
-        t.bit = rb[q] >= 0 ? 0u : (uint32_t)lb[q];
-        for (unsigned i = 0; i < 4; i++) {       // conjugate transpose
-            const cd v = std::conj(op.mat[(i & 1) * 2 + (i >> 1)]);
-            t.f[2 * i] = v.real();
-            t.f[2 * i + 1] = v.imag();
+        flush_run();
+        close();
+        return passes_;
+    }
+
+private:
+    const Circuit& c_;
+    const bool rev_;
+    const unsigned G_;
+    std::vector<SweepOp>& sops_;
+    std::vector<SweepPass> passes_;
+    std::vector<const HOp*> run_;      // diagonal ops since the last mixing one
+    unsigned grads_ = 0;
+    int lane_[SWEEP_LANE_BITS], reg_[8];
+
+    void place(const Stage& st) {
+        // register bits: the qubits mixed first; lane bit 3, whose partners
+        // come by moves, the one mixed least often of the rest
+        std::vector<int> rest(st.tq.begin() + 3, st.tq.end());
+        unsigned uses[64] = {0};
+        std::vector<int> byUse;
+        for (int oi : st.ops) {
+            const int q = sweep_mixes(c_.ops[oi]);
+            if (q < 0) continue;
+            if (!uses[q]++ && std::find(rest.begin(), rest.end(), q) != rest.end()) byUse.push_back(q);
         }
+        for (auto q = rest.rbegin(); q != rest.rend(); ++q) if (!uses[*q]) byUse.push_back(*q);
+        for (unsigned b = 0; b < G_; b++) reg_[b] = byUse[b];
+        std::vector<int> ln(byUse.begin() + G_, byUse.end());
+        std::stable_sort(ln.begin(), ln.end(), [&](int a, int b) { return uses[a] < uses[b]; });
+        for (unsigned b = 0; b < 3; b++) lane_[b] = (int)st.tq[b];
+        for (unsigned b = 0; b < 3; b++) lane_[3 + b] = ln[b];
+    }
+    void open(const Stage& st) {
+        SweepPass p;
+        std::memset(&p.geom, 0, sizeof(p.geom));
+        for (unsigned q : st.tq) p.geom.tileMask |= 1ULL << q;
+        for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) p.geom.lane[b] = (uint8_t)lane_[b];
+        for (unsigned b = 0; b < G_; b++) p.geom.reg[b] = (uint8_t)reg_[b];
+        p.first = sops_.size();
+        grads_ = 0;
+        passes_.push_back(p);
+    }
+    void close() {
+        SweepPass& p = passes_.back();
+        for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) p.geom.laneOut[b] = (uint8_t)lane_[b];
+        for (unsigned b = 0; b < G_; b++) p.geom.regOut[b] = (uint8_t)reg_[b];
+        p.count = (unsigned)(sops_.size() - p.first);
+    }
+    void emit(SweepOp t, const HOp* op) {
+        if (op && rev_ && op->param >= 0) {
+            t.flags |= grads_ & 1u ? SWEEP_GRAD_ODD : SWEEP_GRAD_EVEN;
+            t.row = grads_ / 2;
+            t.slot = (uint32_t)op->param;
+            grads_++;
+        }
+        sops_.push_back(t);
+    }
+    // -tan(a / 2) of the rotation with cosine t.c >= 0 and sine t.g
+    static double shear_t(const SweepOp& t) { return -t.g / (1.0 + t.c); }
+
+    // diagonal ops commute: those with the same slot signs go together
+    void flush_run() {
+        std::vector<std::pair<SweepOp, const HOp*>> ts;
+        for (const HOp* op : run_) ts.emplace_back(translate(*op), op);
+        run_.clear();
+        std::stable_sort(ts.begin(), ts.end(), [](const auto& a, const auto& b) { return a.first.sw < b.first.sw; });
+        for (size_t i = 0; i < ts.size(); i++) {
+            if (i == 0 || ts[i].first.sw != ts[i - 1].first.sw) ts[i].first.flags |= SWEEP_GROUP_FIRST;
+            if (i + 1 == ts.size() || ts[i].first.sw != ts[i + 1].first.sw) ts[i].first.flags |= SWEEP_GROUP_LAST;
+            const uint32_t one = SWEEP_GROUP_FIRST | SWEEP_GROUP_LAST;
+            if ((ts[i].first.flags & one) == one) {
+                ts[i].first.code += SWEEP_DIAG_ONE - SWEEP_DIAG;
+                ts[i].first.c = shear_t(ts[i].first);
+            }
+            emit(ts[i].first, ts[i].second);
+        }
+    }
+    // op (rev: the op that undoes it) in the current layout
+    SweepOp translate(const HOp& op) const {
+        SweepOp t;
+        std::memset(&t, 0, sizeof(t));
+        uint32_t rmask = 0;
+        auto lane_bit = [&](int q) { return (int)(std::find(lane_, lane_ + SWEEP_LANE_BITS, q) - lane_); };
+        auto reg_bit = [&](int q) { return (int)(std::find(reg_, reg_ + G_, q) - reg_); };
+        auto split = [&](uint64_t m) {
+            for (; m; m &= m - 1) {
+                const int q = __builtin_ctzll(m), lb = lane_bit(q), rb = reg_bit(q);
+                if (lb < (int)SWEEP_LANE_BITS) t.lz |= 1u << lb;
+                else if (rb < (int)G_) rmask |= 1u << rb;
+                else t.oz |= 1ULL << q;
+            }
+        };
+        const int q = sweep_mixes(op), rb = q < 0 ? 0 : reg_bit(q);
+        const bool onReg = q >= 0 && rb < (int)G_;
+        if (op.kind == OP_MAT1) {
+            split(op.ctrl);
+            for (uint32_t i = 0; i < (1u << G_); i++) if ((i & rmask) == rmask) t.sw |= 1u << i;
+            t.code = onReg ? SWEEP_MAT_REG + (uint32_t)rb : (uint32_t)SWEEP_MAT_LANE;
+            t.bit = onReg ? 0u : (uint32_t)lane_bit(q);
+            for (unsigned i = 0; i < 4; i++) {       // rev: conjugate transpose
+                const cd v = rev_ ? std::conj(op.mat[(i & 1) * 2 + (i >> 1)]) : op.mat[i];
+                t.f[2 * i] = v.real();
+                t.f[2 * i + 1] = v.imag();
+            }
+            return t;
+        }
+        // A Pauli tensor P is exp(i pi/2 P), and exp(i (theta - pi) P) is
+        // -exp(i theta P): phases common to phi and lambda, which neither <H>
+        // nor a gradient term sees.  So the cosine is taken to be >= 0.
+        const bool tensor = op.kind == OP_PAULI && !op.gadget;
+        double cs = tensor ? 0.0 : std::cos(op.theta), sn = tensor ? 1.0 : std::sin(op.theta);
+        if (rev_) sn = -sn;
+        if (cs < 0) { cs = -cs; sn = -sn; }
+        split(op.kind == OP_PHASE ? op.pmask : op.myz);
+        for (uint32_t i = 0; i < (1u << G_); i++) if (par32(i & rmask)) t.sw |= 1u << i;
+        const uint32_t ss = t.sw != 0;
+        t.c = cs;
+        t.g = sn;                                    // exp(i theta Z..Z)
+        if (q < 0) {
+            t.code = SWEEP_DIAG + ss;
+            return t;
+        }
+        // exp(i theta P) = cos + i sin i^{#Y} (...): imaginary factor for X, real for Y (#Y = 1)
+        const bool y = (op.mxy & op.myz) != 0;
+        if (y) t.g = -sn;
+        if (onReg) {
+            t.code = SWEEP_REG + 4u * (uint32_t)rb;
+            t.c = shear_t(t);
+        } else {
+            t.code = SWEEP_LANE + 4u * (uint32_t)lane_bit(q);
+            if (y) t.lz |= SWEEP_CONST_SIGN;         // the factor is the partner lane's
+        }
+        t.code += (y ? 0u : 2u) + ss;
         return t;
     }
-    // a Pauli tensor P is exp(i pi/2 P) up to a phase common to phi and lambda,
-    // which no gradient term sees
-    const bool tensor = op.kind == OP_PAULI && !op.gadget;
-    const double cs = tensor ? 0.0 : std::cos(op.theta), sn = tensor ? 1.0 : std::sin(op.theta);
-    split(op.kind == OP_PHASE ? op.pmask : op.myz);
-    for (uint32_t i = 0; i < (1u << G); i++) if (par32(i & rmask)) t.sw |= 1u << i;
-    const uint32_t ss = t.sw != 0;
-    t.c = cs;
-    if (op.kind == OP_PHASE || op.mxy == 0) {
-        t.code = SWEEP_DIAG + ss;
-        t.g = -sn;                               // exp(-i theta Z..Z)
-        return t;
-    }
-    // exp(-i theta P) = cos - i sin i^{#Y} (...): imaginary factor for X, real for Y (#Y = 1)
-    const unsigned q = (unsigned)__builtin_ctzll(op.mxy);
-    const bool y = (op.mxy & op.myz) != 0;
-    t.g = y ? sn : -sn;
-    if (rb[q] >= 0) {
-        t.code = SWEEP_REG + 4u * (uint32_t)rb[q];
-    } else {
-        t.code = SWEEP_LANE;
-        t.bit = (uint32_t)lb[q];
-        if (y) t.lz |= SWEEP_CONST_SIGN;         // the factor is the partner lane's
-    }
-    t.code += (y ? 0u : 2u) + ss;
-    return t;
+};
+
+// every tiled stage's passes, their ops in one list on the device
+template <typename R>
+std::vector<std::vector<SweepPass>> sweep_passes(const Circuit& c, const std::vector<Stage>& stages, bool rev,
+                                                 ParamRing& ring, std::vector<SweepOp>& sops, const SweepOp*& dops) {
+    std::vector<std::vector<SweepPass>> passes(stages.size());
+    SweepBuilder<R> b(c, rev, sops);
+    for (size_t si = 0; si < stages.size(); si++)
+        if (stages[si].tiled) passes[si] = b.stage(stages[si]);
+    dops = sops.empty() ? nullptr : static_cast<const SweepOp*>(ring.push(sops.data(), sops.size() * sizeof(SweepOp)));
+    return passes;
 }
 
 // a statevector work state on a stream it does not own
@@ -354,7 +473,30 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
     if (renorm) launch_norm2<R>(st, (const cx<R>*)psi0.amps, psi0.num(), ws, norms);
     hip_check(hipMemcpyAsync(phi.s.amps, psi0.amps, psi0.num() * psi0.amp_bytes(), hipMemcpyDeviceToDevice, st),
               "hipMemcpyAsync");
-    execute(phi.s, plan_for(c, n, psi0.prec));
+    // circuits of ops with a register-tile form run in such passes forward, too
+    if (n >= sweep_min_qubits<R>() && std::all_of(c.ops.begin(), c.ops.end(), sweep_form)) {
+        const std::vector<Stage>& stages = sweep_stages<R>(c, n, psi0.prec, false);
+        ParamRing::Hold hold(phi.s.ring);
+        std::vector<SweepOp> sops;
+        const SweepOp* dops = nullptr;
+        const auto passes = sweep_passes<R>(c, stages, false, phi.s.ring, sops, dops);
+        for (size_t si = 0; si < stages.size(); si++) {
+            if (!stages[si].tiled) {
+                std::vector<HOp> alone;
+                for (int oi : stages[si].ops) alone.push_back(c.ops[oi]);
+                execute_now(phi.s, alone);
+                continue;
+            }
+            for (const SweepPass& p : passes[si]) {
+                ProfScope prof("forward_sweep", st);
+                launch_sweep<R>(st, false, (cx<R>*)phi.s.amps, (cx<R>*)nullptr, n, p.geom, dops + p.first, p.count, 0,
+                                nullptr, 0);
+                hip_check(hipGetLastError(), "forward sweep launch");
+            }
+        }
+    } else {
+        execute(phi.s, plan_for(c, n, psi0.prec));
+    }
     // a unitary circuit keeps the norm; FP32 rounding does not quite.  <H> and
     // every gradient term are quadratic in phi (lambda = H phi), so the
     // forward drift is undone by scaling them by <psi0|psi0> / <phi|phi> at
@@ -440,43 +582,23 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
     };
     if (n >= sweep_min_qubits<R>()) {
         // register-tile passes; stages of one op and ops without such a form alone
-        const std::vector<Stage>& stages = reverse_stages<R>(c, n, psi0.prec);
-        struct Pass { SweepGeom geom; size_t first; unsigned count, grads; };
-        std::vector<SweepOp> sops;
-        std::vector<std::vector<Pass>> passes(stages.size());
-        for (size_t si = 0; si < stages.size(); si++) {
-            if (!stages[si].tiled) continue;
-            const SweepGeom geom = sweep_geom<R>(c, stages[si]);
-            for (int oi : stages[si].ops) {
-                const HOp& op = c.ops[oi];
-                auto& ps = passes[si];
-                if (ps.empty() || (op.param >= 0 && ps.back().grads == SWEEP_MAX_GRADS))
-                    ps.push_back(Pass{geom, sops.size(), 0, 0});
-                SweepOp t = sweep_op<R>(op, geom);
-                if (op.param >= 0) {
-                    const unsigned k = ps.back().grads++;
-                    t.acc = k & 1u ? SWEEP_ACC_SECOND : SWEEP_ACC_FIRST;
-                    t.row = k / 2;
-                    t.slot = (uint32_t)op.param;
-                }
-                ps.back().count++;
-                sops.push_back(t);
-            }
-        }
+        const std::vector<Stage>& stages = sweep_stages<R>(c, n, psi0.prec, true);
         ParamRing::Hold hold(phi.s.ring);        // undo() may push parameters of its own
-        const SweepOp* dops = sops.empty() ? nullptr
-            : static_cast<const SweepOp*>(phi.s.ring.push(sops.data(), sops.size() * sizeof(SweepOp)));
+        std::vector<SweepOp> sops;
+        const SweepOp* dops = nullptr;
+        const auto passes = sweep_passes<R>(c, stages, true, phi.s.ring, sops, dops);
         for (size_t si = 0; si < stages.size(); si++) {
             if (!stages[si].tiled) {
                 for (int oi : stages[si].ops) undo(c.ops[oi]);
                 continue;
             }
-            for (const Pass& p : passes[si]) {
+            for (const SweepPass& p : passes[si]) {
                 ProfScope prof("adjoint_sweep", st);
-                const unsigned nb = launch_sweep<R>(st, a_phi, a_lam, n, p.geom, dops + p.first, p.count, p.grads, rows, stride);
+                const unsigned nb = launch_sweep<R>(st, true, a_phi, a_lam, n, p.geom, dops + p.first, p.count, p.grads,
+                                                    rows, stride);
                 hip_check(hipGetLastError(), "adjoint sweep launch");
                 for (size_t i = p.first; i < p.first + p.count; i++)
-                    if (sops[i].acc != SWEEP_ACC_NONE) nbs[sops[i].slot] = nb;
+                    if (sops[i].flags & (SWEEP_GRAD_EVEN | SWEEP_GRAD_ODD)) nbs[sops[i].slot] = nb;
             }
         }
     } else {

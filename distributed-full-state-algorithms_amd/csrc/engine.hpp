@@ -134,11 +134,11 @@ struct Circuit {
     unsigned cachedNq = 0;
     int cachedPrec = -1;
     Plan cached;
-    // passes of the adjoint's reverse sweep for (revNq, revPrec): stages whose
-    // ops are indices into `ops`
-    unsigned revNq = 0;
-    int revPrec = -1;
-    std::vector<Stage> revStages;
+    // register-tile stages of the adjoint's forward [0] and reverse [1] sweep
+    // for (sweepNq, sweepPrec); their ops are indices into `ops`
+    unsigned sweepNq[2] = {0, 0};
+    int sweepPrec[2] = {-1, -1};
+    std::vector<Stage> sweepStages[2];
     // the adjoint gradient's work states (phi, lambda, their stream), kept for
     // the next call at the same size and precision; freed with the circuit
     std::shared_ptr<AdjointScratch> adj;

@@ -441,97 +441,139 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
     }
 }
 
-// Register-tile pass of the reverse sweep (wave_sweep.hpp).  Gradient terms
-// accumulate per thread in LDS, two gadgets to a row: lanes below 32 keep the
-// first gadget's sum of lanes l and l + 32, the others the second's, so one
-// exchange folds both and a row of 256 doubles serves two gadgets.
+// Register-tile pass (wave_sweep.hpp): REV over phi and lambda, else over phi.
+// Gradient terms accumulate per thread in LDS, two gadgets to a row: lanes
+// below 32 keep the first gadget's sum of lanes l and l + 32, the others the
+// second's, so one exchange folds both and a row of 256 doubles serves two.
 // Three workgroups of four waves per CU (VGPRs and LDS): more waves hide more
 // of the loads and of the scalar work between ops.
-// 24 qubits FP64, 20 layers of 23 ZZ and 24 X gadgets: 35 passes of 375 us (210 us
-// of them the bare loads and stores) against 160 run passes of 197 us and 40
-// diagonal passes of 193 us; 23 qubits FP32 33 of 153 us against 160 of 43-57 and 40 of 48.
-// Bound by the exchanges between lanes and the FP64 arithmetic.
-template <typename R, int G>
+// 20 layers of ZZ and X gadgets, 24 qubits FP64: 35 reverse passes of 315 us (210 us of
+// them the bare loads and stores, against 160 run passes of 197 us and 40
+// diagonal passes of 193 us), 26 forward passes of 147 us (against 19 LDS tile
+// passes of 602 us); 23 qubits FP32: 33 of 135 us and 23 of 46 us.  Bound by
+// vector instructions.  Exchanges through LDS instead of DPP moves and
+// layout changes took 375 us a reverse pass, diagonal gadgets one by one and
+// rotations without shears 336 us.
+template <typename R, int G, bool REV>
 __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
                                                          uint64_t numTiles, SweepGeom geom,
                                                          const SweepOp* __restrict__ ops, unsigned numOps,
                                                          unsigned numGrads, double* __restrict__ rows, uint64_t stride) {
     constexpr int S = 1 << G;
-    __shared__ double acc[SWEEP_MAX_GRADS / 2][BLOCK];
+    __shared__ double acc[REV ? SWEEP_MAX_GRADS / 2 : 1][BLOCK];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const bool upper = lane >= 32u;
-    for (unsigned k = 0; k < (numGrads + 1) / 2; k++) acc[k][tid] = 0;
+    if constexpr (REV)
+        for (unsigned k = 0; k < (numGrads + 1) / 2; k++) acc[k][tid] = 0;
     // The offset of this lane's amplitudes, computed anew for the loads and the
     // stores of a tile: the empty register constraint hides that the two agree,
     // or the compiler would keep all of a tile's addresses alive through its ops.
-    auto lane_offset = [&]() {
+    auto lane_offset = [&](const uint8_t* q) {
         float bits = __builtin_bit_cast(float, lane);
         asm volatile("" : "+v"(bits));
         const uint32_t l = __builtin_bit_cast(uint32_t, bits);
         uint64_t off = 0;
 #pragma unroll
-        for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) off |= (uint64_t)((l >> b) & 1u) << geom.lane[b];
+        for (unsigned b = 0; b < SWEEP_LANE_BITS; b++) off |= (uint64_t)((l >> b) & 1u) << q[b];
         return off;
+    };
+    auto at = [&](uint64_t base, const uint8_t* q, int i) {
+#pragma unroll
+        for (int b = 0; b < G; b++) if ((i >> b) & 1) base |= 1ULL << q[b];
+        return base;
     };
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t first = adjoint_block<R>() * (BLOCK / 64) + wave, step = (uint64_t)gridDim.x * (BLOCK / 64);
-    auto at = [&](uint64_t base, int i) {
-#pragma unroll
-        for (int b = 0; b < G; b++) if ((i >> b) & 1) base |= 1ULL << geom.reg[b];
-        return base;
-    };
     for (uint64_t t = first; t < numTiles; t += step) {
-        const uint64_t base = ins0_mask(t, geom.tileMask), in = lane_offset();
+        const uint64_t base = ins0_mask(t, geom.tileMask), in = lane_offset(geom.lane);
         sweep::Tile<R, S> v;
 #pragma unroll
         for (int i = 0; i < S; i++) {
-            const cx<R> p = adj_ld<R, true>(phi + at(base, i) + in), l = adj_ld<R, true>(lam + at(base, i) + in);
-            v.px[i] = p.x; v.py[i] = p.y; v.lx[i] = l.x; v.ly[i] = l.y;
+            const cx<R> p = adj_ld<R, true>(phi + at(base, geom.reg, i) + in);
+            v.px[i] = p.x; v.py[i] = p.y;
+            if constexpr (REV) {
+                const cx<R> l = adj_ld<R, true>(lam + at(base, geom.reg, i) + in);
+                v.lx[i] = l.x; v.ly[i] = l.y;
+            }
         }
         auto header = [&](unsigned o) {
             SweepOp h;
-            h.code = ops[o].code; h.lz = ops[o].lz; h.sw = ops[o].sw; h.acc = ops[o].acc;
+            h.code = ops[o].code; h.lz = ops[o].lz; h.sw = ops[o].sw; h.flags = ops[o].flags;
             h.oz = ops[o].oz; h.c = ops[o].c; h.g = ops[o].g;
             return h;
         };
         SweepOp hdr = header(0);
-        double held = 0;                                    // the first gadget's term of the current row
+        double held = 0;                                    // the even gadget's term of the current row
+        double dsum = 0, dc = 1, dg = 0;                    // the current diagonal group's sum and factor
         for (unsigned o = 0; o < numOps; o++) {
             const SweepOp next = header(o + 1 < numOps ? o + 1 : o);     // loads while this op runs
-            const double w = sweep::apply<R, G, true>(v, hdr, ops + o, lane, base);
-            if (hdr.acc == SWEEP_ACC_FIRST) {
-                held = w;
-            } else if (hdr.acc == SWEEP_ACC_SECOND) {
-                const double other = __shfl_xor(upper ? held : w, 32, 64);
-                acc[ops[o].row][tid] += (upper ? w : held) + other;
+            // lane and tile part of the sign
+            const uint32_t sb = (par32((lane | SWEEP_CONST_SIGN) & hdr.lz) ^ par64(base & hdr.oz)) << 31;
+            double w;
+            if (hdr.code < SWEEP_LANE) {
+                const bool ss = (hdr.code & 1u) != 0;
+                const double g = sweep::flip(hdr.g, sb);
+                if constexpr (REV) {
+                    if (hdr.flags & SWEEP_GROUP_FIRST)
+                        dsum = ss ? sweep::diag_sum<R, S, true>(v, hdr.sw) : sweep::diag_sum<R, S, false>(v, hdr.sw);
+                }
+                w = sweep::flip(dsum, sb);
+                if (hdr.code >= SWEEP_DIAG_ONE) {
+                    const R T = (R)sweep::flip(hdr.c, sb);
+                    if (ss) sweep::op_diag<R, S, REV, true, true>(v, T, (R)g, hdr.sw);
+                    else sweep::op_diag<R, S, REV, true, false>(v, T, (R)g, hdr.sw);
+                } else {
+                    if (hdr.flags & SWEEP_GROUP_FIRST) { dc = 1; dg = 0; }
+                    const double c = dc * hdr.c - dg * g;
+                    dg = dc * g + dg * hdr.c;
+                    dc = c;
+                    if (hdr.flags & SWEEP_GROUP_LAST) {
+                        if (ss) sweep::op_diag<R, S, REV, false, true>(v, (R)dc, (R)dg, hdr.sw);
+                        else sweep::op_diag<R, S, REV, false, false>(v, (R)dc, (R)dg, hdr.sw);
+                    }
+                }
+            } else {
+                w = sweep::apply<R, G, REV>(v, hdr, ops + o, lane, base, sb);
+            }
+            if constexpr (REV) {
+                if (hdr.flags & SWEEP_GRAD_EVEN) {
+                    held = w;
+                } else if (hdr.flags & SWEEP_GRAD_ODD) {
+                    const double other = __shfl_xor(upper ? held : w, 32, 64);
+                    acc[ops[o].row][tid] += (upper ? w : held) + other;
+                }
             }
             hdr = next;
         }
-        if (numGrads & 1u) {                                // a last gadget on its own
-            const double other = __shfl_xor(upper ? held : 0.0, 32, 64);
-            acc[numGrads / 2][tid] += (upper ? 0.0 : held) + other;
+        if constexpr (REV) {
+            if (numGrads & 1u) {                            // a last gadget on its own
+                const double other = __shfl_xor(upper ? held : 0.0, 32, 64);
+                acc[numGrads / 2][tid] += (upper ? 0.0 : held) + other;
+            }
         }
-        const uint64_t out = lane_offset();
+        const uint64_t out = lane_offset(geom.laneOut);
 #pragma unroll
         for (int i = 0; i < S; i++) {
-            adj_st<R, true>(phi + at(base, i) + out, mk<R>(v.px[i], v.py[i]));
-            adj_st<R, true>(lam + at(base, i) + out, mk<R>(v.lx[i], v.ly[i]));
+            adj_st<R, true>(phi + at(base, geom.regOut, i) + out, mk<R>(v.px[i], v.py[i]));
+            if constexpr (REV) adj_st<R, true>(lam + at(base, geom.regOut, i) + out, mk<R>(v.lx[i], v.ly[i]));
         }
     }
-    // workgroup sums: gadget 2 k in the lower, 2 k + 1 in the upper lanes of row k
-    unsigned k = 0;
-    for (unsigned o = 0; o < numOps; o++) {
-        if (ops[o].acc == SWEEP_ACC_NONE) continue;
-        const double a = acc[k / 2][tid];
-        double im = upper == ((k & 1u) != 0) ? a : 0.0, dummy = 0;
-        block_sum2(im, dummy);
-        if (tid == 0) {
-            double* row = rows + stride * ops[o].slot + 2 * blockIdx.x;
-            row[0] = 0;
-            row[1] = im;
+    if constexpr (REV) {
+        // workgroup sums: gadget 2 k in the lower, 2 k + 1 in the upper lanes of row k
+        unsigned k = 0;
+        for (unsigned o = 0; o < numOps; o++) {
+            if (!(ops[o].flags & (SWEEP_GRAD_EVEN | SWEEP_GRAD_ODD))) continue;
+            const double a = acc[k / 2][tid];
+            double im = upper == ((k & 1u) != 0) ? a : 0.0, dummy = 0;
+            block_sum2(im, dummy);
+            if (tid == 0) {
+                double* row = rows + stride * ops[o].slot + 2 * blockIdx.x;
+                row[0] = 0;
+                row[1] = im;
+            }
+            __syncthreads();    // block_sum2's wave partials are reused by the next gadget
+            k++;
         }
-        __syncthreads();    // block_sum2's wave partials are reused by the next gadget
-        k++;
     }
 }
 
@@ -846,18 +888,19 @@ unsigned launch_adjoint_qrun(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq,
     return nb;
 }
 
-// three workgroups per CU, each wave on every (12 * CUs)-th tile; never more than
+// three (rev) or four workgroups per CU, as many as its registers allow; never more than
 // red_blocks(2^nq) rows (a workgroup's four tiles hold 2^11 amplitudes or more)
 template <typename R>
-unsigned launch_sweep(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom, const SweepOp* dops,
-                      unsigned numOps, unsigned numGrads, double* rows, uint64_t stride) {
-    constexpr unsigned G = sweep_reg_bits<R>(), M = SWEEP_LANE_BITS + G;
-    if (nq < M || numOps == 0 || numGrads > SWEEP_MAX_GRADS || (unsigned)__builtin_popcountll(geom.tileMask) != M)
+unsigned launch_sweep(hipStream_t s, bool rev, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom,
+                      const SweepOp* dops, unsigned numOps, unsigned numGrads, double* rows, uint64_t stride) {
+    const unsigned M = SWEEP_LANE_BITS + sweep_reg_bits<R>(rev);
+    if (nq < M || numOps == 0 || numGrads > (rev ? SWEEP_MAX_GRADS : 0) ||
+        (unsigned)__builtin_popcountll(geom.tileMask) != M)
         fail(FSA_ERR_INTERNAL, "register-tile pass of unsupported shape");
     const uint64_t numTiles = 1ULL << (nq - M);
-    const unsigned nb = (unsigned)std::min<uint64_t>((numTiles + BLOCK / 64 - 1) / (BLOCK / 64), 768);
-    hipLaunchKernelGGL((k_wave_sweep<R, (int)G>), dim3(nb), dim3(BLOCK), 0, s, phi, lam, numTiles, geom, dops, numOps,
-                       numGrads, rows, stride);
+    const unsigned nb = (unsigned)std::min<uint64_t>((numTiles + BLOCK / 64 - 1) / (BLOCK / 64), rev ? 768 : 1024);
+    auto* kern = rev ? k_wave_sweep<R, (int)sweep_reg_bits<R>(true), true> : k_wave_sweep<R, (int)sweep_reg_bits<R>(false), false>;
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(BLOCK), 0, s, phi, lam, numTiles, geom, dops, numOps, numGrads, rows, stride);
     return nb;
 }
 
@@ -973,8 +1016,8 @@ void launch_f32_to_f64(hipStream_t s, const cx<float>* in, cx<double>* out, uint
     template void launch_inner<R>(hipStream_t, const cx<R>*, const cx<R>*, uint64_t, double*, double*);       \
     template unsigned launch_adjoint_step<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointStepDev&,       \
                                              double*, uint64_t);                                                \
-    template unsigned launch_sweep<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const SweepGeom&, const SweepOp*,    \
-                                      unsigned, unsigned, double*, uint64_t);                                   \
+    template unsigned launch_sweep<R>(hipStream_t, bool, cx<R>*, cx<R>*, unsigned, const SweepGeom&,              \
+                                      const SweepOp*, unsigned, unsigned, double*, uint64_t);                   \
     template unsigned launch_adjoint_diag<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointDiagDev&,       \
                                              double*, uint64_t);                                                \
     template unsigned launch_adjoint_qrun<R>(hipStream_t, cx<R>*, cx<R>*, unsigned, const AdjointQubitRunDev&,   \

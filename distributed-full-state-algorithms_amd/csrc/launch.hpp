@@ -113,44 +113,51 @@ template <typename R> constexpr int sweep_bits() { return sizeof(R) == 8 ? 2 : 4
 // outside the tile; lz / oz are the lane and outside parts of its Z mask
 // (matrices: control mask), sw has bit i set where slot i's parity is odd
 // (matrices: where slot i's controls are set).  Bit 6 of lz is a constant sign.
-enum SweepCode : uint32_t {       // imag and ss (sw != 0) select the form: + 2 imag + ss
-    SWEEP_DIAG = 0,      // v' = v (c + i g s), s = +-1 by parity (imag always 0 here)
-    SWEEP_LANE = 4,      // Pauli string with its X/Y qubit on lane bit `bit`:
-    SWEEP_REG = 8,       // ... on register bit B (+ 4 B): v' = c v + (imag ? i g : g) s w, w the partner
-    SWEEP_MAT_LANE = 28, // 2x2 matrix f (row-major) on lane bit `bit`
-    SWEEP_MAT_REG = 29,  // ... on register bit B (+ B)
-};
+enum SweepCode : uint32_t {
+    SWEEP_DIAG = 0,      // (+ ss) diagonal gadget of a group: v' = v (c + i g s), s = +-1 by parity
+    SWEEP_DIAG_ONE = 2,  // (+ ss) a group of one: the same with c = -tan(a/2), g = sin a (shears)
+    SWEEP_LANE = 4,      // (+ 4 b + 2 imag + ss) Pauli string with its X/Y qubit on lane bit b < 4:
+                         // v' = c v + (imag ? i g : g) s w, w the partner
+    SWEEP_REG = 20,      // (+ 4 B + 2 imag + ss) ... on register bit B, c and g as in SWEEP_DIAG_ONE
+    SWEEP_SWAP = 40,     // (+ 5 (l - 4) + B) lane bit l = 4, 5 and register bit B change places
+    SWEEP_MAT_LANE = 50, // 2x2 matrix f (row-major) on lane bit `bit`
+    SWEEP_MAT_REG = 51,  // (+ B) ... on register bit B
+};                       // ss: sw != 0
 constexpr uint32_t SWEEP_CONST_SIGN = 64;
-// Gradient terms: of a pass's gadgets, the ones numbered 2 k and 2 k + 1 share
-// accumulator row k (see k_wave_sweep)
-enum SweepAcc : uint32_t { SWEEP_ACC_NONE = 0, SWEEP_ACC_FIRST = 1, SWEEP_ACC_SECOND = 2 };
+// Flags of an op.  Of a pass's gradient terms, numbers 2 k and 2 k + 1 share
+// accumulator row k (see k_wave_sweep).  Consecutive diagonal gadgets with the
+// same sw form a group, which costs one multiplication of the tile.
+enum SweepFlags : uint32_t { SWEEP_GRAD_EVEN = 1, SWEEP_GRAD_ODD = 2, SWEEP_GROUP_FIRST = 4, SWEEP_GROUP_LAST = 8 };
 struct SweepOp {
-    uint32_t code, lz, sw, acc;
+    uint32_t code, lz, sw, flags;
     uint64_t oz;
     double c, g;
     uint32_t bit;
-    uint32_t row;        // accumulator row (SECOND)
+    uint32_t row;        // accumulator row (SWEEP_GRAD_ODD)
     uint32_t slot;       // row slot of its gradient term
     uint32_t pad;
     double f[8];
 };
 constexpr unsigned SWEEP_LANE_BITS = 6;
-// register bits: 64 VGPRs of amplitudes for phi and lambda
-template <typename R> constexpr unsigned sweep_reg_bits() { return sizeof(R) == 8 ? 3u : 4u; }
-// Smallest states that the passes take.  Smaller ones give a pass one to four
+// register bits: 64 VGPRs of amplitudes (rev: of phi and lambda together)
+template <typename R> constexpr unsigned sweep_reg_bits(bool rev) { return (sizeof(R) == 8 ? 4u : 5u) - (rev ? 1u : 0u); }
+// Smallest states that the passes take.  Smaller ones give a pass one or two
 // waves, which run its ops one after another, and the run kernels' launches of
-// a few us each are no slower: 20 layers of ZZ and X gadgets take 1.21 ms either way at 10
-// qubits FP64, and in FP32 1.33 against 1.20 ms at 10, 1.68 against 1.70 at 12.
+// a few us each are no slower.  20 layers of ZZ and X gadgets, ms per gradient,
+// passes against run kernels: 1.05 / 1.22 at 10 qubits FP64; in FP32 1.42 / 1.70 at
+// 12, while at 10 and 11 an earlier form of the passes took 1.33 / 1.20 and
+// 1.49 / 1.39.
 template <typename R> constexpr unsigned sweep_min_qubits() { return sizeof(R) == 8 ? 10u : 12u; }
 constexpr unsigned SWEEP_MAX_GRADS = 46;     // gradient terms of a pass: two per 2 KiB row of LDS
 struct SweepGeom {
     uint64_t tileMask;
-    uint8_t lane[8], reg[8];                 // qubits of the lane and register bits
+    uint8_t lane[8], reg[8];                 // qubits of the lane and register bits as the tile is loaded
+    uint8_t laneOut[8], regOut[8];           // ... and as it is stored
 };
-// one pass over phi and lambda; returns the number of workgroups (rows per slot)
+// one pass over phi and lambda (rev) or phi alone; returns the number of workgroups (rows per slot)
 template <typename R>
-unsigned launch_sweep(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom, const SweepOp* dops,
-                      unsigned numOps, unsigned numGrads, double* rows, uint64_t stride);
+unsigned launch_sweep(hipStream_t s, bool rev, cx<R>* phi, cx<R>* lam, unsigned nq, const SweepGeom& geom,
+                      const SweepOp* dops, unsigned numOps, unsigned numGrads, double* rows, uint64_t stride);
 
 // ---- init / copy / conversion ------------------------------------------------
 template <typename R>

@@ -8,7 +8,10 @@
 // them back: no LDS traffic for the amplitudes and no barriers, so the waves
 // of a SIMD drift apart and one's loads and stores hide behind another's
 // arithmetic.  Ops mix amplitudes along one register bit (arithmetic only) or
-// one lane bit (partners from lane l ^ bit); diagonal ops need no tile qubit.
+// one of lane bits 0-3 (partners by DPP moves); a qubit on lane bit 4 or 5
+// first changes places with one on a register bit (one instruction per word of
+// a pair of slots), so the tile may be stored in another layout than it was
+// loaded in.  Diagonal ops need no tile qubit.
 // Controls and Z factors may sit anywhere: their parity splits into a part of
 // the lane, a part of the slot (one bit per slot, prepared by the host) and a
 // part fixed for the tile.
@@ -39,7 +42,7 @@ __device__ __forceinline__ uint32_t slot_sign(uint32_t sw, int i) { return (sw <
 template <int ID, typename R>
 __device__ __forceinline__ void pin(R& v) { asm volatile("" : "+v"(v) : "n"(ID)); }
 
-// v' = c v + (i g or g) w: IMAG picks the imaginary factor
+// v' = c v + (i g or g) w: IMAG picks the imaginary factor (lane bits, diagonal groups)
 template <bool IMAG, typename R>
 __device__ __forceinline__ void rot(R& x, R& y, R wx, R wy, R c, R g) {
     const R ox = x, oy = y;
@@ -50,6 +53,16 @@ __device__ __forceinline__ void rot(R& x, R& y, R wx, R wy, R c, R g) {
         x = c * ox + g * wx;
         y = c * oy + g * wy;
     }
+}
+
+// The rotation (x, y) -> (cos a x - sin a y, sin a x + cos a y) as three shears,
+// T = -tan(a / 2) and g = sin a: three multiply-adds in place instead of two
+// and two products, and |T| <= 1 because the host takes a from (-pi/2, pi/2].
+template <typename R>
+__device__ __forceinline__ void shear(R& x, R& y, R T, R g) {
+    x += T * y;
+    y += g * x;
+    x += T * y;
 }
 
 // Im or Re of conj(l) p in FP64
@@ -64,78 +77,184 @@ struct Tile {
     R px[S], py[S], lx[S], ly[S];
 };
 
-// e^{-i theta Z..Z}: v' = v (c + i g s), s = +-1 by parity (g carries the lane's sign)
-template <typename R, int S, bool REV, bool SS>
-__device__ __forceinline__ void op_diag(Tile<R, S>& t, R c, R g, uint32_t sw, double& sum) {
-    pin<SS>(c);
-    pin<SS>(g);
+// the value of lane l ^ (1 << BIT): DPP moves on the vector unit (quad_perm,
+// row_half_mirror after quad_perm, row_ror:8), so the exchange does not go
+// through the LDS crossbar
+template <int BIT>
+__device__ __forceinline__ uint32_t lane_xor32(uint32_t v) {
+#if defined(__AMDGCN__)
+    if constexpr (BIT == 0) return __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, true);
+    if constexpr (BIT == 1) return __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, true);
+    if constexpr (BIT == 2) {
+        v = __builtin_amdgcn_update_dpp(v, v, 0x1B, 0xf, 0xf, true);
+        return __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, true);
+    }
+    return __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, true);
+#else
+    return (uint32_t)__shfl_xor(v, 1 << BIT, 64);
+#endif
+}
+template <int BIT>
+__device__ __forceinline__ float lane_xor(float v) {
+    return __builtin_bit_cast(float, lane_xor32<BIT>(__builtin_bit_cast(uint32_t, v)));
+}
+template <int BIT>
+__device__ __forceinline__ double lane_xor(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(double, (uint64_t)lane_xor32<BIT>((uint32_t)u) |
+                                          ((uint64_t)lane_xor32<BIT>((uint32_t)(u >> 32)) << 32));
+}
+
+// lane bit L (4 or 5) and the register bit that tells a from b change places:
+// a's upper half goes to b's lower one and back, one instruction per word
+template <int L>
+__device__ __forceinline__ void exchange32(uint32_t& a, uint32_t& b) {
+#if defined(__AMDGCN__)
+    if constexpr (L == 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0]; b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0]; b = r[1];
+    }
+#else
+    const bool up = (threadIdx.x >> L) & 1u;
+    const uint32_t x = (uint32_t)__shfl_xor(up ? a : b, 1 << L, 64);
+    if (up) a = x;
+    else b = x;
+#endif
+}
+template <int L>
+__device__ __forceinline__ void exchange(float& a, float& b) {
+    uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+    exchange32<L>(x, y);
+    a = __builtin_bit_cast(float, x);
+    b = __builtin_bit_cast(float, y);
+}
+template <int L>
+__device__ __forceinline__ void exchange(double& a, double& b) {
+    const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+    uint32_t xl = (uint32_t)x, xh = (uint32_t)(x >> 32), yl = (uint32_t)y, yh = (uint32_t)(y >> 32);
+    exchange32<L>(xl, yl);
+    exchange32<L>(xh, yh);
+    a = __builtin_bit_cast(double, (uint64_t)xl | ((uint64_t)xh << 32));
+    b = __builtin_bit_cast(double, (uint64_t)yl | ((uint64_t)yh << 32));
+}
+
+// the tile's sum of Im conj(lambda) phi, slots signed by sw
+template <typename R, int S, bool SS>
+__device__ __forceinline__ double diag_sum(Tile<R, S>& t, uint32_t sw) {
     double s[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < S; i++) {
-        const R gi = SS ? flip(g, slot_sign(sw, i)) : g;
-        if constexpr (REV) {
-            pin<SS>(t.lx[i]);
-            pin<SS>(t.ly[i]);
-            const double w = term<true>(t.lx[i], t.ly[i], t.px[i], t.py[i]);
-            s[i & 1] += SS ? flip(w, slot_sign(sw, i)) : w;
-            rot<true>(t.lx[i], t.ly[i], t.lx[i], t.ly[i], c, gi);
-        }
-        rot<true>(t.px[i], t.py[i], t.px[i], t.py[i], c, gi);
+        pin<SS>(t.lx[i]);
+        pin<SS>(t.ly[i]);
+        const double w = term<true>(t.lx[i], t.ly[i], t.px[i], t.py[i]);
+        s[i & 1] += SS ? flip(w, slot_sign(sw, i)) : w;
     }
-    sum = s[0] + s[1];
+    return s[0] + s[1];
 }
 
-// the X/Y qubit on register bit B: pairs (i, j = i | 1 << B)
+// diagonal factors: v' = v (c + i g s), s the slot's sign
+// (ONE: c is the shear coefficient T of a single gadget)
+template <typename R, int S, bool REV, bool ONE, bool SS>
+__device__ __forceinline__ void op_diag(Tile<R, S>& t, R c, R g, uint32_t sw) {
+    pin<2 + 2 * ONE + SS>(c);
+    pin<2 + 2 * ONE + SS>(g);
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+        const R gi = SS ? flip(g, slot_sign(sw, i)) : g;
+        if constexpr (ONE) {
+            const R Ti = SS ? flip(c, slot_sign(sw, i)) : c;
+            if constexpr (REV) shear(t.lx[i], t.ly[i], Ti, gi);
+            shear(t.px[i], t.py[i], Ti, gi);
+        } else {
+            if constexpr (REV) rot<true>(t.lx[i], t.ly[i], t.lx[i], t.ly[i], c, gi);
+            rot<true>(t.px[i], t.py[i], t.px[i], t.py[i], c, gi);
+        }
+    }
+}
+
+// The X/Y qubit on register bit B: pairs (i, j = i | 1 << B), each two plane
+// rotations.  IMAG (X): v_i' = c v_i + i g v_j and back mix (x_i, y_j) and
+// (x_j, y_i); the two amplitudes have the same sign.  Otherwise (Y)
+// v_i' = c v_i - g v_j, v_j' = c v_j + g v_i mix (x_i, x_j) and (y_i, y_j); the
+// signs are opposite, and g is taken with that of i, the second's partner.
 template <typename R, int S, bool REV, int B, bool IMAG, bool SS>
-__device__ __forceinline__ void op_reg(Tile<R, S>& t, R c, R g, uint32_t sw, double& sum) {
-    pin<8 + 4 * B + 2 * IMAG + SS>(c);
-    pin<8 + 4 * B + 2 * IMAG + SS>(g);
+__device__ __forceinline__ void op_reg(Tile<R, S>& t, R T, R g, uint32_t sw, double& sum) {
+    constexpr int ID = 8 + 4 * B + 2 * IMAG + SS;
+    pin<ID>(T);
+    pin<ID>(g);
     double s[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < S; i++) {
         if (i & (1 << B)) continue;
         const int j = i | (1 << B);
-        // an amplitude takes its partner's sign
-        const R gi = SS ? flip(g, slot_sign(sw, i)) : g, gj = SS ? flip(g, slot_sign(sw, j)) : g;
+        const R gi = SS ? flip(g, slot_sign(sw, i)) : g, Ti = SS ? flip(T, slot_sign(sw, i)) : T;
         if constexpr (REV) {
-            pin<8 + 4 * B + 2 * IMAG + SS>(t.lx[i]);
-            pin<8 + 4 * B + 2 * IMAG + SS>(t.ly[i]);
-            pin<8 + 4 * B + 2 * IMAG + SS>(t.lx[j]);
-            pin<8 + 4 * B + 2 * IMAG + SS>(t.ly[j]);
+            pin<ID>(t.lx[i]);
+            pin<ID>(t.ly[i]);
+            pin<ID>(t.lx[j]);
+            pin<ID>(t.ly[j]);
+            // an amplitude takes its partner's sign
             const double wi = term<IMAG>(t.lx[i], t.ly[i], t.px[j], t.py[j]);
             const double wj = term<IMAG>(t.lx[j], t.ly[j], t.px[i], t.py[i]);
             s[0] += SS ? flip(wi, slot_sign(sw, j)) : wi;
             s[1] += SS ? flip(wj, slot_sign(sw, i)) : wj;
-            const R ax = t.lx[i], ay = t.ly[i];
-            rot<IMAG>(t.lx[i], t.ly[i], t.lx[j], t.ly[j], c, gj);
-            rot<IMAG>(t.lx[j], t.ly[j], ax, ay, c, gi);
+            if constexpr (IMAG) {
+                shear(t.lx[i], t.ly[j], Ti, gi);
+                shear(t.lx[j], t.ly[i], Ti, gi);
+            } else {
+                shear(t.lx[i], t.lx[j], Ti, gi);
+                shear(t.ly[i], t.ly[j], Ti, gi);
+            }
         }
-        const R ax = t.px[i], ay = t.py[i];
-        rot<IMAG>(t.px[i], t.py[i], t.px[j], t.py[j], c, gj);
-        rot<IMAG>(t.px[j], t.py[j], ax, ay, c, gi);
+        if constexpr (IMAG) {
+            shear(t.px[i], t.py[j], Ti, gi);
+            shear(t.px[j], t.py[i], Ti, gi);
+        } else {
+            shear(t.px[i], t.px[j], Ti, gi);
+            shear(t.py[i], t.py[j], Ti, gi);
+        }
     }
     sum = s[0] + s[1];
 }
 
-// the X/Y qubit on a lane bit: partners from lane l ^ m (g carries the partner lane's sign)
-template <typename R, int S, bool REV, bool IMAG, bool SS>
-__device__ __forceinline__ void op_lane(Tile<R, S>& t, int m, R c, R g, uint32_t sw, double& sum) {
-    pin<4 + 2 * IMAG + SS>(c);
-    pin<4 + 2 * IMAG + SS>(g);
+// the X/Y qubit on lane bit B: partners from lane l ^ (1 << B) (g carries the partner lane's sign)
+template <typename R, int S, bool REV, int B, bool IMAG, bool SS>
+__device__ __forceinline__ void op_lane(Tile<R, S>& t, R c, R g, uint32_t sw, double& sum) {
+    pin<100 + 4 * B + 2 * IMAG + SS>(c);
+    pin<100 + 4 * B + 2 * IMAG + SS>(g);
     double s[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < S; i++) {
         const R gi = SS ? flip(g, slot_sign(sw, i)) : g;
-        const R wx = __shfl_xor(t.px[i], m, 64), wy = __shfl_xor(t.py[i], m, 64);
+        const R wx = lane_xor<B>(t.px[i]), wy = lane_xor<B>(t.py[i]);
         if constexpr (REV) {
             const double w = term<IMAG>(t.lx[i], t.ly[i], wx, wy);
             s[i & 1] += SS ? flip(w, slot_sign(sw, i)) : w;
-            const R ux = __shfl_xor(t.lx[i], m, 64), uy = __shfl_xor(t.ly[i], m, 64);
+            const R ux = lane_xor<B>(t.lx[i]), uy = lane_xor<B>(t.ly[i]);
             rot<IMAG>(t.lx[i], t.ly[i], ux, uy, c, gi);
         }
         rot<IMAG>(t.px[i], t.py[i], wx, wy, c, gi);
     }
     sum = s[0] + s[1];
+}
+
+// lane bit L and register bit B change places
+template <typename R, int S, bool REV, int L, int B>
+__device__ __forceinline__ void op_swap(Tile<R, S>& t) {
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+        if (i & (1 << B)) continue;
+        const int j = i | (1 << B);
+        exchange<L>(t.px[i], t.px[j]);
+        exchange<L>(t.py[i], t.py[j]);
+        if constexpr (REV) {
+            exchange<L>(t.lx[i], t.lx[j]);
+            exchange<L>(t.ly[i], t.ly[j]);
+        }
+    }
 }
 
 template <typename R>
@@ -181,12 +300,14 @@ __device__ __forceinline__ void op_mat_lane(Tile<R, S>& t, int m, bool set, cons
     }
 }
 
-// Applies op to the tile (hdr: its fields up to g, already loaded) and returns
-// the lane's part of its gradient term.
+// Applies an op other than a diagonal gadget to the tile (hdr: its fields up to
+// g, already loaded; sb: sign bit of its lane and tile part) and returns the
+// lane's part of its gradient term.
 template <typename R, int G, bool REV>
 __device__ __forceinline__ double apply(Tile<R, 1 << G>& t, const SweepOp& hdr, const SweepOp* __restrict__ op,
-                                        uint32_t lane, uint64_t base) {
+                                        uint32_t lane, uint64_t base, uint32_t sb) {
     constexpr int S = 1 << G;
+    const uint32_t sw = hdr.sw;
     if (hdr.code >= SWEEP_MAT_LANE) {
         if ((base & hdr.oz) != hdr.oz) return 0;             // a control outside the tile is 0
         R f[8];
@@ -195,36 +316,42 @@ __device__ __forceinline__ double apply(Tile<R, 1 << G>& t, const SweepOp& hdr, 
         const bool on = (lane & hdr.lz) == hdr.lz;
         const uint32_t bit = op->bit;
         switch (hdr.code) {
-        case SWEEP_MAT_LANE: op_mat_lane<R, S, REV>(t, 1 << bit, ((lane >> bit) & 1u) != 0, f, hdr.sw, on); break;
-        case SWEEP_MAT_REG + 0: if constexpr (G > 0) op_mat_reg<R, S, REV, 0>(t, f, hdr.sw, on); break;
-        case SWEEP_MAT_REG + 1: if constexpr (G > 1) op_mat_reg<R, S, REV, 1>(t, f, hdr.sw, on); break;
-        case SWEEP_MAT_REG + 2: if constexpr (G > 2) op_mat_reg<R, S, REV, 2>(t, f, hdr.sw, on); break;
-        case SWEEP_MAT_REG + 3: if constexpr (G > 3) op_mat_reg<R, S, REV, 3>(t, f, hdr.sw, on); break;
-        case SWEEP_MAT_REG + 4: if constexpr (G > 4) op_mat_reg<R, S, REV, 4>(t, f, hdr.sw, on); break;
+        case SWEEP_MAT_LANE: op_mat_lane<R, S, REV>(t, 1 << bit, ((lane >> bit) & 1u) != 0, f, sw, on); break;
+        case SWEEP_MAT_REG + 0: if constexpr (G > 0) op_mat_reg<R, S, REV, 0>(t, f, sw, on); break;
+        case SWEEP_MAT_REG + 1: if constexpr (G > 1) op_mat_reg<R, S, REV, 1>(t, f, sw, on); break;
+        case SWEEP_MAT_REG + 2: if constexpr (G > 2) op_mat_reg<R, S, REV, 2>(t, f, sw, on); break;
+        case SWEEP_MAT_REG + 3: if constexpr (G > 3) op_mat_reg<R, S, REV, 3>(t, f, sw, on); break;
+        case SWEEP_MAT_REG + 4: if constexpr (G > 4) op_mat_reg<R, S, REV, 4>(t, f, sw, on); break;
         default: break;
         }
         return 0;
     }
-    const R c = (R)hdr.c;
-    // lane and tile part of the sign
-    const uint32_t sb = (par32((lane | SWEEP_CONST_SIGN) & hdr.lz) ^ par64(base & hdr.oz)) << 31;
-    const R g = flip((R)hdr.g, sb);
-    const uint32_t sw = hdr.sw;
+    // a shear coefficient (register bits) changes sign with g, a cosine does not
+    const R g = flip((R)hdr.g, sb), c = hdr.code >= SWEEP_REG ? flip((R)hdr.c, sb) : (R)hdr.c;
     double sum = 0;
     switch (hdr.code) {
-    case SWEEP_DIAG: op_diag<R, S, REV, false>(t, c, g, sw, sum); break;
-    case SWEEP_DIAG + 1: op_diag<R, S, REV, true>(t, c, g, sw, sum); break;
-    case SWEEP_LANE: op_lane<R, S, REV, false, false>(t, 1 << op->bit, c, g, sw, sum); break;
-    case SWEEP_LANE + 1: op_lane<R, S, REV, false, true>(t, 1 << op->bit, c, g, sw, sum); break;
-    case SWEEP_LANE + 2: op_lane<R, S, REV, true, false>(t, 1 << op->bit, c, g, sw, sum); break;
-    case SWEEP_LANE + 3: op_lane<R, S, REV, true, true>(t, 1 << op->bit, c, g, sw, sum); break;
-#define FSA_SWEEP_B(BV)                                                                                          \
+#define FSA_SWEEP_FORMS(OP, BASE, BV)                                             \
+    case BASE + 4 * BV: OP<R, S, REV, BV, false, false>(t, c, g, sw, sum); break; \
+    case BASE + 4 * BV + 1: OP<R, S, REV, BV, false, true>(t, c, g, sw, sum); break; \
+    case BASE + 4 * BV + 2: OP<R, S, REV, BV, true, false>(t, c, g, sw, sum); break; \
+    case BASE + 4 * BV + 3: OP<R, S, REV, BV, true, true>(t, c, g, sw, sum); break;
+    FSA_SWEEP_FORMS(op_lane, SWEEP_LANE, 0) FSA_SWEEP_FORMS(op_lane, SWEEP_LANE, 1)
+    FSA_SWEEP_FORMS(op_lane, SWEEP_LANE, 2) FSA_SWEEP_FORMS(op_lane, SWEEP_LANE, 3)
+    FSA_SWEEP_FORMS(op_reg, SWEEP_REG, 0) FSA_SWEEP_FORMS(op_reg, SWEEP_REG, 1) FSA_SWEEP_FORMS(op_reg, SWEEP_REG, 2)
+#undef FSA_SWEEP_FORMS
+    // register bits that not every tile has
+#define FSA_SWEEP_FORMS(BV)                                                                                      \
     case SWEEP_REG + 4 * BV: if constexpr (G > BV) op_reg<R, S, REV, BV, false, false>(t, c, g, sw, sum); break; \
     case SWEEP_REG + 4 * BV + 1: if constexpr (G > BV) op_reg<R, S, REV, BV, false, true>(t, c, g, sw, sum); break; \
     case SWEEP_REG + 4 * BV + 2: if constexpr (G > BV) op_reg<R, S, REV, BV, true, false>(t, c, g, sw, sum); break; \
     case SWEEP_REG + 4 * BV + 3: if constexpr (G > BV) op_reg<R, S, REV, BV, true, true>(t, c, g, sw, sum); break;
-    FSA_SWEEP_B(0) FSA_SWEEP_B(1) FSA_SWEEP_B(2) FSA_SWEEP_B(3) FSA_SWEEP_B(4)
-#undef FSA_SWEEP_B
+    FSA_SWEEP_FORMS(3) FSA_SWEEP_FORMS(4)
+#undef FSA_SWEEP_FORMS
+#define FSA_SWEEP_SWAP(LV, BV) \
+    case SWEEP_SWAP + 5 * (LV - 4) + BV: if constexpr (G > BV) op_swap<R, S, REV, LV, BV>(t); break;
+    FSA_SWEEP_SWAP(4, 0) FSA_SWEEP_SWAP(4, 1) FSA_SWEEP_SWAP(4, 2) FSA_SWEEP_SWAP(4, 3) FSA_SWEEP_SWAP(4, 4)
+    FSA_SWEEP_SWAP(5, 0) FSA_SWEEP_SWAP(5, 1) FSA_SWEEP_SWAP(5, 2) FSA_SWEEP_SWAP(5, 3) FSA_SWEEP_SWAP(5, 4)
+#undef FSA_SWEEP_SWAP
     default: break;
     }
     return flip(sum, sb);

@@ -1,4 +1,4 @@
-"""Register-tile passes of the adjoint's reverse sweep (wave_sweep.hpp): on the
+"""Register-tile passes of the adjoint (wave_sweep.hpp): on the
 CPU stand-in under AddressSanitizer and on the GPU, against the oracle's adjoint.
 
 The circuit holds every op the passes take, on every kind of bit (lane,
@@ -14,7 +14,8 @@ import pytest
 from test_emu_kernels import _run, _unitary, _write_op, drive  # noqa: F401
 
 
-def circuit(rng, n, layers):
+def circuit(rng, n, layers, forms=False):
+    """forms: only ops with a register-tile form (the forward sweep takes them too)"""
     ang = lambda: float(rng.uniform(0, 6.3))
     ops = []
     for layer in range(layers):
@@ -25,13 +26,14 @@ def circuit(rng, n, layers):
         q = [int(x) for x in rng.permutation(n)]
         ops.append(("pauliGadget", (q[:3], [1, 3, 3], ang())))
         ops.append(("pauliGadget", (q[3:6], [3, 2, 3], ang())))
-        ops.append(("pauliGadget", (q[:3], [1, 2, 3], ang())))
+        if not forms:
+            ops.append(("pauliGadget", (q[:3], [1, 2, 3], ang())))
         ops.append(("oneTargGate", (q[0], _unitary(rng, 2))))
         for c in (1, 2):
             for s in range(0, n - c, 3):
                 ops.append(("manyCtrlOneTargGate", (q[s + 1:s + 1 + c], q[s], _unitary(rng, 2))))
         ops.append(("pauliGadget", (q[:4], [3, 3, 3, 3], ang())))
-        if layer:
+        if layer and not forms:
             ops.append(("manyTargGate", (q[2:5], _unitary(rng, 8))))
     return ops
 
@@ -67,10 +69,10 @@ def oracle_adjoint(orc, psi, ops, coeffs, paulis):
 
 
 # rounding of L ops on unit vectors: L * a few eps on <H> and on the gradient's norm
-@pytest.mark.parametrize("n,prec,tol", [(10, 0, 1e-12), (12, 0, 1e-12), (12, 1, 2e-5)])
-def test_sweep_passes_on_cpu(drive, orc, tmp_path, n, prec, tol):  # noqa: F811
+@pytest.mark.parametrize("n,prec,forms,tol", [(10, 0, False, 1e-12), (12, 0, True, 1e-12), (12, 1, True, 2e-5)])
+def test_sweep_passes_on_cpu(drive, orc, tmp_path, n, prec, forms, tol):  # noqa: F811
     rng = np.random.default_rng(900 + n + prec)
-    ops = circuit(rng, n, 2)
+    ops = circuit(rng, n, 2, forms)
     coeffs, paulis = observable(rng, n)
     psi = np.zeros(1 << n, complex)
     psi[0] = 1
@@ -86,17 +88,20 @@ def test_sweep_passes_on_cpu(drive, orc, tmp_path, n, prec, tol):  # noqa: F811
     out = _run(drive, ["adjoint", path, prec])
     assert out["expec_abs_err"] <= tol and out["grad_rel_err"] <= tol, out
     assert out["adjoint_sweep"] >= 2, out
+    assert ("forward_sweep" in out) == forms, out
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("forms", [False, True])
 @pytest.mark.parametrize("n", [10, 11, 12, 13, 18])
-def test_sweep_passes_on_gpu(orc, n):
+def test_sweep_passes_on_gpu(orc, n, forms):
     import __graft_entry__ as ge
 
     fsa = ge.load_package()
     rng = np.random.default_rng(950 + n)
-    ops = circuit(rng, n, 3)
-    ops.insert(20, ("swapGate", (0, n - 1)))
+    ops = circuit(rng, n, 3, forms)
+    if not forms:
+        ops.insert(20, ("swapGate", (0, n - 1)))
     ops.insert(50, ("pauliTensor", ([1, 3, n - 1], [2, 3, 3])))
     ops.insert(70, ("pauliTensor", ([2, n - 2], [3, 3])))
     ops.insert(30, ("phaseGadget", ([0, 5, n - 2], 0.7)))
@@ -114,6 +119,7 @@ def test_sweep_passes_on_gpu(orc, n):
         fsa.profile_enable(False)
         if n >= (10 if prec == "fp64" else 12):
             assert launches["adjoint_sweep"][0] >= 2, launches
+            assert ("forward_sweep" in launches) == forms, launches
         assert abs(e - expec) <= tol * np.abs(coeffs).sum()
         assert np.linalg.norm(g - grads) <= tol * np.linalg.norm(grads), (prec, np.linalg.norm(g - grads))
         # new angles, same passes; then the first ones again, bit for bit
