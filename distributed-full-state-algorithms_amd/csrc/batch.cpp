@@ -26,9 +26,7 @@ int batch_occupancy(int tb, int m);
 template <typename R>
 bool launch_batch(hipStream_t s, int tb, int m, unsigned grid, const BatchJob* jobs, unsigned numJobs,
                   const BatchStage* stages, const TileOp* items, const cx<double>* mats, const PauliTermDev* terms,
-                  const double* params, cx<R>* arena, double* res, unsigned* counter);
-
-constexpr unsigned MAX_STAGE_GRADS_HOST = 512;   // LDS gradient accumulators per pass (kernels_batch.hip)
+                  const double* params, unsigned numParams, double* cs, cx<R>* arena, double* res, unsigned* counter);
 
 struct BatchEntry {
     unsigned n = 0;
@@ -149,7 +147,7 @@ struct BlobBuilder {
                 const int oi = s.ops[ii];
                 const HOp& op = ops[oi];
                 TileOp t = translate_item<double>(op, pos, bs.tileMask, mats);
-                if (op.kind == OP_GRAD && ngrad == MAX_STAGE_GRADS_HOST) {
+                if (op.kind == OP_GRAD && ngrad == BATCH_STAGE_GRADS) {
                     // close the pass and continue the same ops in a new one on the same tiles
                     bs.nitems = (uint32_t)(items.size() - bs.item0);
                     stages.push_back(bs);
@@ -214,6 +212,8 @@ void build_impl(Batch& b) {
         BatchJob J{};
         J.n = e.n;
         J.resident = resident ? 1u : 0u;
+        auto mark = [&](int i) { J.item[i] = (uint32_t)bb.items.size(); J.mat[i] = (uint32_t)bb.mats.size(); };
+        mark(0);
         bb.add_plan(fwd, fsign, e.n, sp, numJobs, false, J.fwd0, J.nfwd);
         if (!resident && J.nfwd == 0) {
             // the first forward pass creates |0..0> in the arena, so there is always one
@@ -225,7 +225,9 @@ void build_impl(Batch& b) {
             J.nfwd = 1;
             bb.stages.push_back(bs);
         }
+        mark(1);
         bb.add_plan(rev, rsign, e.n, sp, numJobs, true, J.rev0, J.nrev);
+        mark(2);
         J.term0 = (uint32_t)bb.terms.size();
         J.nterm = (uint32_t)e.terms.size();
         bb.terms.insert(bb.terms.end(), e.terms.begin(), e.terms.end());
@@ -272,7 +274,8 @@ void build_impl(Batch& b) {
     dev_alloc((void**)&b.blob, blobBytes, "the batch plans");
     b.resDoubles = 2ULL * (numJobs + b.totalParams) + numJobs;   // <H>, gradients, <phi|phi>
     dev_alloc((void**)&b.dres, b.resDoubles * sizeof(double), "the batch results");
-    dev_alloc((void**)&b.dparams, std::max<size_t>(1, b.totalParams) * sizeof(double), "the batch angles");
+    // the angles, then their cosines and sines
+    dev_alloc((void**)&b.dparams, std::max<size_t>(1, b.totalParams) * 3 * sizeof(double), "the batch angles");
     dev_alloc((void**)&b.dcounter, 256, "the batch counter");
     hip_check(hipHostMalloc((void**)&b.hres, b.resDoubles * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
     hip_check(hipHostMalloc((void**)&b.hparams, std::max<size_t>(1, b.totalParams) * sizeof(double),
@@ -309,6 +312,7 @@ void run_impl(Batch& b, double* expecs, double* grads) {
                                         reinterpret_cast<const TileOp*>(b.blob + b.offItems),
                                         reinterpret_cast<const cx<double>*>(b.blob + b.offMats),
                                         reinterpret_cast<const PauliTermDev*>(b.blob + b.offTerms), b.dparams,
+                                        b.totalParams, b.dparams + b.totalParams,
                                         static_cast<cx<R>*>(b.arena), b.dres, b.dcounter);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(b.stream, &g);

@@ -173,6 +173,9 @@ struct BatchStage {
     uint32_t pad;
 };
 
+// gradient items per stage: their per-wave sums share the LDS left by the tiles
+constexpr uint32_t BATCH_STAGE_GRADS = 96;
+
 struct BatchJob {
     uint64_t phi, lam;    // element offsets of phi / lambda in the arena (unused when resident)
     uint32_t n;           // qubits
@@ -183,6 +186,7 @@ struct BatchJob {
     uint32_t out;         // result slot of <H> (two doubles)
     uint32_t slot0, nslot;// result slots of the job's gradients, zeroed at the start
     uint32_t nrm;         // result double that receives <phi|phi> after the forward plan
+    uint32_t item[3], mat[3];  // first item / matrix element of the forward and the reverse plan, and the end
 };
 
 }  // namespace fsa

@@ -15,9 +15,11 @@
 // (results are bit-identical run to run) and there is no inter-workgroup wait:
 // each workgroup leaves the loop as soon as the counter passes the last job.
 //
-// Gadget angles are read from `params` at run time (item field param, sign in
-// f[6], i^#Y in f[4..5]), so new angles only need a copy into that array:
-// the launch itself can be captured once in a graph and replayed.
+// Gadget angles are read from `params` at run time, so new angles only need a
+// copy into that array: the launch itself can be captured once in a graph and
+// replayed.  A first small kernel turns them into cosines and sines (item field
+// param picks a pair, f[6] its sign, f[4..5] i^#Y); formed per item by every
+// thread they took about as long as the item's LDS sweep.
 #include "launch.hpp"
 #include "tile_ops.hpp"
 
@@ -60,12 +62,10 @@ __device__ __forceinline__ void bsum2(double& vr, double& vi, double* red) {
     vi = b;
 }
 
-// gadget factors from the run-time angle (forward: sign +1, inverse: -1)
-__device__ __forceinline__ void bind_param(TileOp& op, const double* __restrict__ params) {
+// gadget factors from the run-time angle's cosine and sine (forward: sign +1, inverse: -1)
+__device__ __forceinline__ void bind_param(TileOp& op, const double* __restrict__ cs) {
     if (op.param == NO_PARAM) return;
-    const double t = op.f[6] * params[op.param];
-    double s, c;
-    sincos(t, &s, &c);
+    const double c = cs[2 * (size_t)op.param], s = op.f[6] * cs[2 * (size_t)op.param + 1];
     if (op.kind == OP_PAULI) {            // exp(i t P): this = cos t, other = i sin t * i^#Y
         op.f[0] = c; op.f[1] = 0.0;
         op.f[2] = -s * op.f[5]; op.f[3] = s * op.f[4];
@@ -75,10 +75,10 @@ __device__ __forceinline__ void bind_param(TileOp& op, const double* __restrict_
     }
 }
 
-// <lambda|P|phi> over one tile: sum_l conj(lam_l) i^#Y (-1)^{par(k & myz)} phi_k, k = l ^ mxy
+// Im <lambda|P|phi> over one tile: sum_l conj(lam_l) i^#Y (-1)^{par(k & myz)} phi_k, k = l ^ mxy
 template <typename R, int TB>
-__device__ __forceinline__ void grad_partial(const cx<R>* phi, const cx<R>* lam, uint32_t T, uint64_t base,
-                                             const TileOp& op, double& vr, double& vi) {
+__device__ __forceinline__ double grad_partial(const cx<R>* phi, const cx<R>* lam, uint32_t T, uint64_t base,
+                                               const TileOp& op) {
     const uint32_t bp = par64(base & op.gmask);
     double ar = 0, ai = 0;
     for (uint32_t l = threadIdx.x; l < T; l += TB) {
@@ -88,67 +88,88 @@ __device__ __forceinline__ void grad_partial(const cx<R>* phi, const cx<R>* lam,
         ar += sg * ((double)x.x * (double)y.x + (double)x.y * (double)y.y);
         ai += sg * ((double)x.x * (double)y.y - (double)x.y * (double)y.x);
     }
-    vr = op.f[0] * ar - op.f[1] * ai;
-    vi = op.f[0] * ai + op.f[1] * ar;
+    return op.f[0] * ai + op.f[1] * ar;
 }
 
 // A gradient item fused with the inverse gadget after it (same Pauli masks):
 // one sweep over the pairs (l, l ^ mxy) of both tiles accumulates the item's
-// <lambda|P|phi> terms (as grad_partial) and applies the gadget `o` to phi and
-// lambda with the arithmetic of tile_apply's OP_PAULI / OP_PHASE.
-template <typename R, int TB>
-__device__ __forceinline__ void grad_apply(cx<R>* phi, cx<R>* lam, uint32_t T, uint64_t base, const TileOp& g,
-                                           const TileOp& o, double& vr, double& vi) {
+// Im <lambda|P|phi> terms (as grad_partial) and applies the gadget `o` to phi
+// and lambda with the arithmetic of tile_apply's OP_PAULI / OP_PHASE.  ROWS:
+// amplitudes per thread of a full tile, whose loads are then issued together.
+template <typename R, int TB, int ROWS>
+__device__ __forceinline__ double grad_apply(cx<R>* phi, cx<R>* lam, uint32_t T, uint64_t base, const TileOp& g,
+                                             const TileOp& o) {
     const uint32_t bp = par64(base & g.gmask);
     const uint32_t lxy = g.lmask, lyz = g.lmask2;
+    const uint32_t tid = threadIdx.x;
     double ar = 0, ai = 0;
     auto term = [&](const cx<R>& x, const cx<R>& y, uint32_t k) {   // conj(x) y (-1)^{par(k & myz)}
         const double sg = (bp ^ par32(k & lyz)) ? -1.0 : 1.0;
         ar += sg * ((double)x.x * (double)y.x + (double)x.y * (double)y.y);
         ai += sg * ((double)x.x * (double)y.y - (double)x.y * (double)y.x);
     };
+    // n pieces of work, N of them per thread when the tile is full: B at a time
+    auto sweep = [&](uint32_t n, auto count, auto batch, auto load, auto store) {
+        constexpr int N = decltype(count)::value, B = N < decltype(batch)::value ? N : decltype(batch)::value;
+        if (N > 1 && n == (uint32_t)N * TB) {
+#pragma unroll
+            for (int i0 = 0; i0 < N; i0 += B) {
+                cx<R> v[B > 0 ? B : 1][4];
+#pragma unroll
+                for (int i = 0; i < B; i++) load(tid + (uint32_t)(i0 + i) * TB, v[i]);
+#pragma unroll
+                for (int i = 0; i < B; i++) store(tid + (uint32_t)(i0 + i) * TB, v[i]);
+            }
+            return;
+        }
+        cx<R> v[4];
+        for (uint32_t j = tid; j < n; j += TB) { load(j, v); store(j, v); }
+    };
+    auto load1 = [&](uint32_t l, cx<R>* v) { v[0] = phi[l]; v[1] = lam[l]; };
     if (o.kind == OP_PHASE) {
         const cx<double> f0 = ldc<double>(o.f, 0), f1 = ldc<double>(o.f, 1);
         const uint32_t bq = par64(base & o.gmask);
-        for (uint32_t l = threadIdx.x; l < T; l += TB) {
-            const cx<R> x = lam[l], y = phi[l];
-            term(x, y, l);
+        sweep(T, std::integral_constant<int, ROWS>{}, std::integral_constant<int, 8>{}, load1, [&](uint32_t l, cx<R>* v) {
+            term(v[1], v[0], l);
             const cx<double> f = (bq ^ par32(l & o.lmask)) ? f1 : f0;
-            phi[l] = dn<R>(cmul(up<double>(y), f));
-            lam[l] = dn<R>(cmul(up<double>(x), f));
-        }
+            phi[l] = dn<R>(cmul(up<double>(v[0]), f));
+            lam[l] = dn<R>(cmul(up<double>(v[1]), f));
+        });
     } else {
         const cx<double> th = ldc<double>(o.f, 0), fe = ldc<double>(o.f, 1);
         const cx<double> fo = mk<double>(-fe.x, -fe.y);
         const uint32_t bq = par64(base & o.gmask);
         if (lxy == 0) {
-            for (uint32_t l = threadIdx.x; l < T; l += TB) {
-                const cx<R> x = lam[l], y = phi[l];
-                term(x, y, l);
+            sweep(T, std::integral_constant<int, ROWS>{}, std::integral_constant<int, 8>{}, load1, [&](uint32_t l, cx<R>* v) {
+                term(v[1], v[0], l);
                 const cx<double> f = (bq ^ par32(l & o.lmask2)) ? fo : fe;
-                const cx<double> yd = up<double>(y), xd = up<double>(x);
+                const cx<double> yd = up<double>(v[0]), xd = up<double>(v[1]);
                 phi[l] = dn<R>(cfma(cmul(th, yd), f, yd));
                 lam[l] = dn<R>(cfma(cmul(th, xd), f, xd));
-            }
+            });
         } else {
             const unsigned hb = 31u - (unsigned)__builtin_clz(lxy);
-            for (uint32_t j = threadIdx.x; j < (T >> 1); j += TB) {
-                const uint32_t i0 = ins0_32(j, hb), i1 = i0 ^ lxy;
-                const cx<R> p0 = phi[i0], p1 = phi[i1], l0 = lam[i0], l1 = lam[i1];
-                term(l0, p1, i1);
-                term(l1, p0, i0);
-                const cx<double> f0 = (bq ^ par32(i0 & o.lmask2)) ? fo : fe;
-                const cx<double> f1 = (bq ^ par32(i1 & o.lmask2)) ? fo : fe;
-                const cx<double> q0 = up<double>(p0), q1 = up<double>(p1), m0 = up<double>(l0), m1 = up<double>(l1);
-                phi[i0] = dn<R>(cfma(cmul(th, q0), f1, q1));
-                phi[i1] = dn<R>(cfma(cmul(th, q1), f0, q0));
-                lam[i0] = dn<R>(cfma(cmul(th, m0), f1, m1));
-                lam[i1] = dn<R>(cfma(cmul(th, m1), f0, m0));
-            }
+            sweep(T >> 1, std::integral_constant<int, ROWS / 2>{}, std::integral_constant<int, 4>{},
+                  [&](uint32_t j, cx<R>* v) {
+                      const uint32_t i0 = ins0_32(j, hb), i1 = i0 ^ lxy;
+                      v[0] = phi[i0]; v[1] = phi[i1]; v[2] = lam[i0]; v[3] = lam[i1];
+                  },
+                  [&](uint32_t j, cx<R>* v) {
+                      const uint32_t i0 = ins0_32(j, hb), i1 = i0 ^ lxy;
+                      term(v[2], v[1], i1);
+                      term(v[3], v[0], i0);
+                      const cx<double> f0 = (bq ^ par32(i0 & o.lmask2)) ? fo : fe;
+                      const cx<double> f1 = (bq ^ par32(i1 & o.lmask2)) ? fo : fe;
+                      const cx<double> q0 = up<double>(v[0]), q1 = up<double>(v[1]);
+                      const cx<double> m0 = up<double>(v[2]), m1 = up<double>(v[3]);
+                      phi[i0] = dn<R>(cfma(cmul(th, q0), f1, q1));
+                      phi[i1] = dn<R>(cfma(cmul(th, q1), f0, q0));
+                      lam[i0] = dn<R>(cfma(cmul(th, m0), f1, m1));
+                      lam[i1] = dn<R>(cfma(cmul(th, m1), f0, m0));
+                  });
         }
     }
-    vr = g.f[0] * ar - g.f[1] * ai;
-    vi = g.f[0] * ai + g.f[1] * ar;
+    return g.f[0] * ai + g.f[1] * ar;
 }
 
 // lambda_j = sum_t f_t (-1)^{par(k & myz_t)} phi_k, k = j ^ mxy_t, for j in [j0, j0 + T);
@@ -177,45 +198,45 @@ __device__ __forceinline__ void apply_terms(const cx<R>* phiAll, cx<R>* lamOut, 
     }
 }
 
-// Gradient items of one stage accumulate in LDS (gacc, indexed by the item's
-// p[0] = its index among the stage's gradient items) over the tiles a
-// workgroup processes, and are written out once per stage (flush_grads).
-constexpr uint32_t MAX_STAGE_GRADS = 512;
+// Gradient items of one stage accumulate in LDS, one sum per wave (gacc[wave *
+// BATCH_STAGE_GRADS + g], g = the item's p[0], its index among the stage's
+// gradient items), over the tiles a workgroup processes, and are added up and
+// written out once per stage (flush_grads): no barrier of their own.
 
 // the items of one stage on the LDS tile(s); OP_GRAD items add their tile sum
-// into gacc (tiles in a fixed order)
+// into gacc (tiles in a fixed order).  REV: lambda's tile follows phi's, and an
+// item runs on both as on one tile of twice the size (none of its masks reach
+// the bit that tells them apart).
 template <typename R, int TB, bool REV, int ROWS>
-__device__ __forceinline__ void run_items(cx<R>* phi, cx<R>* lam, uint32_t T, uint64_t base,
-                                          const TileOp* __restrict__ items, uint32_t i0, uint32_t ni,
-                                          const cx<double>* __restrict__ mats, const double* __restrict__ params,
-                                          double* gacc, double* red, bool firstTile) {
+__device__ __forceinline__ void run_items(cx<R>* phi, uint32_t T, uint64_t base, const TileOp* __restrict__ items,
+                                          uint32_t i0, uint32_t ni, const cx<double>* __restrict__ mats,
+                                          const double* __restrict__ cs, double* gacc, bool firstTile) {
+    cx<R>* lam = phi + T;
     for (uint32_t i = i0; i < i0 + ni; i++) {
         TileOp op = items[i];
         if (REV && op.kind == OP_GRAD) {
-            double vr, vi;
+            double v;
             const bool fused = op.k == 1u;  // the next item is this gadget's inverse
             if (fused) {
                 TileOp inv = items[i + 1];
-                bind_param(inv, params);
-                grad_apply<R, TB>(phi, lam, T, base, op, inv, vr, vi);
+                bind_param(inv, cs);
+                v = grad_apply<R, TB, ROWS>(phi, lam, T, base, op, inv);
                 i++;
             } else {
-                grad_partial<R, TB>(phi, lam, T, base, op, vr, vi);
+                v = grad_partial<R, TB>(phi, lam, T, base, op);
             }
-            bsum2<TB>(vr, vi, red);
-            if (threadIdx.x == 0) {
-                double* r = gacc + 2 * op.p[0];
-                if (firstTile) { r[0] = vr; r[1] = vi; }
-                else { r[0] += vr; r[1] += vi; }
+            v = bwave_sum(v);
+            if ((threadIdx.x & 63u) == 0) {
+                double* r = gacc + (threadIdx.x >> 6) * BATCH_STAGE_GRADS + op.p[0];
+                *r = firstTile ? v : *r + v;
             }
             if (fused) __syncthreads();     // the tiles were written (a gradient sum alone only reads them)
             continue;
         }
-        bind_param(op, params);
+        bind_param(op, cs);
         // full tiles (T = ROWS * TB) load batches of four pairs before updating them
         // (one workgroup per CU: registers to spare)
-        tile_apply<R, TB, 1, 1, double, ROWS, 4>(phi, T, base, op, mats);
-        if (REV) tile_apply<R, TB, 1, 1, double, ROWS, 4>(lam, T, base, op, mats);
+        tile_apply<R, TB, 1, 1, double, REV ? 2 * ROWS : ROWS, 4>(phi, REV ? 2 * T : T, base, op, mats);
         __syncthreads();
     }
 }
@@ -227,28 +248,34 @@ __device__ __forceinline__ void flush_grads(const BatchStage& st, const TileOp* 
     __syncthreads();
     for (uint32_t i = st.item0 + threadIdx.x; i < st.item0 + st.nitems; i += TB) {
         if (items[i].kind == OP_GRAD) {
-            const uint32_t g = items[i].p[0];
-            const size_t slot = items[i].mat_off;
-            res[2 * slot] = gacc[2 * g];
-            res[2 * slot + 1] = gacc[2 * g + 1];
+            double v = 0;
+#pragma unroll
+            for (int w = 0; w < TB / 64; w++) v += gacc[w * BATCH_STAGE_GRADS + items[i].p[0]];
+            res[2 * (size_t)items[i].mat_off + 1] = v;
         }
     }
     __syncthreads();
 }
 
+// Bound by the phases of each item's LDS sweep: eight waves read, combine and
+// write a tile between two barriers (a 4096-amplitude sweep takes about 2800
+// clocks, its LDS traffic alone 1160).  256 jobs of 10-15 qubits, 50-300 gates:
+// 10.9 ms with angles turned into factors by every thread of every item, phi and
+// lambda swept one after the other and a workgroup reduction per gradient term;
+// 9.2 ms now.
 template <typename R, int TB, int M>
 __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs, unsigned numJobs,
                                               const BatchStage* __restrict__ stages,
                                               const TileOp* __restrict__ items, const cx<double>* __restrict__ mats,
                                               const PauliTermDev* __restrict__ terms,
-                                              const double* __restrict__ params, cx<R>* __restrict__ arena,
+                                              const double* __restrict__ cs, cx<R>* __restrict__ arena,
                                               double* __restrict__ res, unsigned* __restrict__ counter) {
     constexpr uint32_t TMAX = 1u << M;
     constexpr uint32_t KMAX = TMAX / TB > 0 ? TMAX / TB : 1;
     __shared__ cx<R> lds[2 * TMAX];
     __shared__ uint64_t offHi[KMAX];
     __shared__ double red[2 * (TB / 64)];
-    __shared__ double gacc[2 * MAX_STAGE_GRADS];
+    __shared__ double gacc[(TB / 64) * BATCH_STAGE_GRADS];
     __shared__ unsigned jobIdx;
     const uint32_t tid = threadIdx.x;
 
@@ -259,6 +286,17 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
         const unsigned jx = jobIdx;
         if (jx >= numJobs) break;
         const BatchJob J = jobs[jx];
+        // Reads one word of every cache line of the job's items and matrices, all
+        // in flight at once, so that the scalar loads of each item later find
+        // them in L2 (64 12-qubit jobs: 1.60 -> 1.36 ms).
+        double seen = 0;
+        auto touch = [&](const void* first, size_t bytes) {
+            const double* p = static_cast<const double*>(first);
+            for (size_t i = (size_t)tid * 8; i < bytes / 8; i += TB * 8) seen += p[i];
+        };
+        touch(items + J.item[0], (J.item[2] - J.item[0]) * sizeof(TileOp));
+        touch(mats + J.mat[0], (J.mat[2] - J.mat[0]) * sizeof(cx<double>));
+        if (seen == 1.2345678e-300) red[0] = seen;   // keeps the loads; red is free here
 
         if (J.resident) {
             // ---- whole job in LDS: phi = lds[0, T), lambda = lds[T, 2T)
@@ -268,8 +306,7 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
             for (uint32_t l = tid; l < T; l += TB) phi[l] = mk<R>(l == 0 ? (R)1 : (R)0, (R)0);
             __syncthreads();
             for (uint32_t s = J.fwd0; s < J.fwd0 + J.nfwd; s++)
-                run_items<R, TB, false, KMAX>(phi, lam, T, 0, items, stages[s].item0, stages[s].nitems, mats, params, gacc,
-                                        red, true);
+                run_items<R, TB, false, KMAX>(phi, T, 0, items, stages[s].item0, stages[s].nitems, mats, cs, gacc, true);
             double er = 0, ei = 0, nn = 0, nz = 0;
             apply_terms<R, TB>(phi, lam, 0, T, terms + J.term0, J.nterm, er, ei, nn);
             bsum2<TB>(er, ei, red);
@@ -282,7 +319,7 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
             __syncthreads();
             for (uint32_t s = J.rev0; s < J.rev0 + J.nrev; s++) {
                 const BatchStage st = stages[s];
-                run_items<R, TB, true, KMAX>(phi, lam, T, 0, items, st.item0, st.nitems, mats, params, gacc, red, true);
+                run_items<R, TB, true, KMAX>(phi, T, 0, items, st.item0, st.nitems, mats, cs, gacc, true);
                 flush_grads<TB>(st, items, gacc, res);
             }
             continue;
@@ -344,8 +381,7 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
             if (1 < numTiles) load(1);
             for (uint64_t t = 0; t < numTiles; t++) {
                 const uint64_t base = pdep64(t, outMask);
-                run_items<R, TB, REV, KMAX>(lds, lds + TMAX, T, base, items, st.item0, st.nitems, mats, params, gacc,
-                                      red, t == 0);
+                run_items<R, TB, REV, KMAX>(lds, T, base, items, st.item0, st.nitems, mats, cs, gacc, t == 0);
                 __syncthreads();   // the last item may be a gradient sum still reading other rows
                 // Each thread writes its own rows of tile t back and fills them
                 // with tile t + 1; the wait makes tile t + 1's loads land before the
@@ -405,8 +441,16 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
     }
 }
 
-__global__ void k_batch_reset(unsigned* counter) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) counter[0] = 0u;
+// resets the job counter and turns the angles into cosines and sines
+__global__ void k_batch_prepare(unsigned* counter, const double* __restrict__ params, unsigned numParams,
+                                double* __restrict__ cs) {
+    const unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0) counter[0] = 0u;
+    if (p >= numParams) return;
+    double s, c;
+    sincos(params[p], &s, &c);
+    cs[2 * (size_t)p] = c;
+    cs[2 * (size_t)p + 1] = s;
 }
 
 }  // namespace
@@ -434,12 +478,13 @@ int batch_occupancy(int tb, int m) {
 template <typename R>
 bool launch_batch(hipStream_t s, int tb, int m, unsigned grid, const BatchJob* jobs, unsigned numJobs,
                   const BatchStage* stages, const TileOp* items, const cx<double>* mats, const PauliTermDev* terms,
-                  const double* params, cx<R>* arena, double* res, unsigned* counter) {
-    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, counter);
+                  const double* params, unsigned numParams, double* cs, cx<R>* arena, double* res, unsigned* counter) {
+    hipLaunchKernelGGL(k_batch_prepare, dim3(std::max(1u, (numParams + 255) / 256)), dim3(256), 0, s, counter, params,
+                       numParams, cs);
 #define FSA_BL(TBV, MV)                                                                                    \
     if (tb == TBV && m == MV) {                                                                            \
         hipLaunchKernelGGL((k_batch<R, TBV, MV>), dim3(grid), dim3(TBV), 0, s, jobs, numJobs, stages, items, \
-                           mats, terms, params, arena, res, counter);                                      \
+                           mats, terms, cs, arena, res, counter);                                          \
         return true;                                                                                       \
     }
     FSA_BL(256, 10) FSA_BL(256, 11) FSA_BL(256, 12) FSA_BL(512, 10) FSA_BL(512, 11) FSA_BL(512, 12)
@@ -453,10 +498,10 @@ template int batch_max_bits<float>();
 template int batch_occupancy<double>(int, int);
 template int batch_occupancy<float>(int, int);
 template bool launch_batch<double>(hipStream_t, int, int, unsigned, const BatchJob*, unsigned, const BatchStage*,
-                                   const TileOp*, const cx<double>*, const PauliTermDev*, const double*,
-                                   cx<double>*, double*, unsigned*);
+                                   const TileOp*, const cx<double>*, const PauliTermDev*, const double*, unsigned,
+                                   double*, cx<double>*, double*, unsigned*);
 template bool launch_batch<float>(hipStream_t, int, int, unsigned, const BatchJob*, unsigned, const BatchStage*,
-                                  const TileOp*, const cx<double>*, const PauliTermDev*, const double*, cx<float>*,
-                                  double*, unsigned*);
+                                  const TileOp*, const cx<double>*, const PauliTermDev*, const double*, unsigned,
+                                  double*, cx<float>*, double*, unsigned*);
 
 }  // namespace fsa

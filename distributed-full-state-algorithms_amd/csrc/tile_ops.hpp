@@ -69,7 +69,28 @@ __device__ __forceinline__ void tile_matk(cx<R>* s, uint32_t T, const TileOp& op
     constexpr int OUTMAX = sizeof(C) == 8 ? 8 : 16;
     constexpr int OUT = D < OUTMAX ? D : OUTMAX;
     // whole groups per thread, written in place; a full tile has >= TB groups only when D <= OUT
-    if constexpr (D <= OUT) if (groups >= (uint32_t)TB) {
+    if constexpr (D <= 8) if (groups >= (uint32_t)TB) {
+        // The inputs of a group are read together, then its outputs are formed
+        // row by row: one LDS wait per group, and a row of the matrix is
+        // contiguous, so its scalar loads are wide and run ahead by rows.
+        // (Column by column, with one input and one matrix column at a time,
+        // every input cost an LDS wait and a scalar wait.)
+        for (uint32_t g = tid; g < groups; g += TB) {
+            const uint32_t b = ins0_mask32(g, tm);
+            cx<C> x[D];
+#pragma unroll
+            for (int l = 0; l < D; l++) x[l] = up<C>(s[b | FSA_OFF((uint32_t)l)]);
+#pragma unroll
+            for (int o = 0; o < D; o++) {
+                cx<C> acc = mk<C>(0, 0);
+#pragma unroll
+                for (int l = 0; l < D; l++) acc = cfma(acc, mat[o * D + l], x[l]);
+                s[b | FSA_OFF((uint32_t)o)] = dn<R>(acc);
+            }
+        }
+        return;
+    }
+    if constexpr (D > 8 && D <= OUT) if (groups >= (uint32_t)TB) {
         for (uint32_t g = tid; g < groups; g += TB) {
             const cx<C>* m = mat;
             const uint32_t b = ins0_mask32(g, tm);
@@ -495,9 +516,10 @@ __device__ __forceinline__ void tile_apply(cx<R>* s, uint32_t T, uint64_t base, 
         const uint32_t b0 = 1u << op.p[0], b1 = 1u << op.p[1];
         for (uint32_t j = tid; j < (T >> 2); j += TB) {
             uint32_t i = ins0_mask32(j, b0 | b1);
-            cx<R> x = s[i | b0], y = s[i | b1];
-            s[i | b0] = y;
-            s[i | b1] = x;
+            // by components: copies of the structs went through private memory
+            const R ax = s[i | b0].x, ay = s[i | b0].y, bx = s[i | b1].x, by = s[i | b1].y;
+            s[i | b0] = mk<R>(bx, by);
+            s[i | b1] = mk<R>(ax, ay);
         }
         return;
     }
