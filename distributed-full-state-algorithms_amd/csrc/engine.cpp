@@ -134,61 +134,107 @@ static void dump_schedule(const char* path, const std::vector<HOp>& ops, const s
 // qubits this gives 771 passes over six seeds of the generator against 823
 // for the plain scan from the low qubits (128 against 138 for the default
 // seed).
+//
+// Planning is host time that every flush and every new circuit pays, so the
+// scans run over compact records (an op's masks and nothing else), a scan that
+// only counts stops once it can take no more ops or can no longer beat the
+// best count, and equal seeds are tried once; the stages are the ones the plain
+// form of the search finds.
+namespace {
+
+struct SchedRec {
+    uint64_t nd, touch;
+    uint64_t blockNd;    // what it blocks for non-diagonal use when deferred
+    int op;
+    bool fits;
+};
+
+struct SchedScan {
+    unsigned m;          // tile qubits
+    uint64_t full;       // a blocked mask that stops every op (the union of all touched qubits)
+
+    bool takes(const SchedRec& r, uint64_t blockedNd, uint64_t blockedAll, uint64_t& tile) const {
+        if (!r.fits || (r.nd & blockedAll) || (r.touch & blockedNd)) return false;
+        const uint64_t nt = tile | r.nd;
+        if (nt != tile && (unsigned)__builtin_popcountll(nt) > m) return false;
+        tile = nt;
+        return true;
+    }
+    // ops that a scan of list[0, n) from this tile takes; 0 or more if that is at most `best`
+    size_t count(const SchedRec* list, size_t n, uint64_t tile, size_t best) const {
+        uint64_t blockedNd = 0, blockedAll = 0;
+        size_t taken = 0;
+        for (size_t r = 0; r < n; r++) {
+            if (takes(list[r], blockedNd, blockedAll, tile)) {
+                taken++;
+                continue;
+            }
+            blockedNd |= list[r].blockNd;
+            blockedAll |= list[r].touch;
+            if (blockedNd == full || taken + (n - 1 - r) <= best) break;
+        }
+        return taken;
+    }
+    // splits list[0, n) into the ops taken and the rest; returns the tile
+    uint64_t split(const std::vector<SchedRec>& list, size_t n, uint64_t tile, std::vector<SchedRec>& taken,
+                   std::vector<SchedRec>& rest) const {
+        uint64_t blockedNd = 0, blockedAll = 0;
+        taken.clear();
+        rest.clear();
+        size_t r = 0;
+        for (; r < n && blockedNd != full; r++) {
+            if (takes(list[r], blockedNd, blockedAll, tile)) {
+                taken.push_back(list[r]);
+                continue;
+            }
+            rest.push_back(list[r]);
+            blockedNd |= list[r].blockNd;
+            blockedAll |= list[r].touch;
+        }
+        rest.insert(rest.end(), list.begin() + r, list.begin() + n);
+        return tile;
+    }
+};
+
+}  // namespace
+
 std::vector<Stage> schedule(const std::vector<HOp>& ops, unsigned nq, SchedParams sp) {
     std::vector<Stage> stages;
     const uint64_t lowMask = sp.low >= 64 ? ~0ULL : ((1ULL << sp.low) - 1ULL);
     const unsigned freeSlots = sp.m - sp.low;
-    auto fits = [&](const HOp& op) {
-        return op.tileable && (unsigned)__builtin_popcountll(op.nd & ~lowMask) <= freeSlots;
-    };
     const unsigned seeds = env_u("FSA_SCHED_SEEDS", 16);
     const unsigned look = env_u("FSA_SCHED_LOOK", 16);
     const size_t window = std::max(1u, env_u("FSA_SCHED_WINDOW", 256));
-    // one scan of the first `limit` ops of `list` from a seeded tile: the
-    // tile it ends with, the ops it takes (in order) and the rest
-    auto scan = [&](const std::vector<int>& list, size_t limit, uint64_t tile, std::vector<int>& tk,
-                    std::vector<int>& df) {
-        uint64_t blockedNd = 0, blockedAll = 0;
-        tk.clear();
-        df.clear();
-        const size_t n = std::min(limit, list.size());
-        for (size_t r = 0; r < n; r++) {
-            const int i = list[r];
-            const HOp& op = ops[i];
-            bool take = false;
-            if (fits(op) && !(op.nd & blockedAll) && !(op.touch & blockedNd)) {
-                uint64_t nt = tile | op.nd;
-                if ((unsigned)__builtin_popcountll(nt) <= sp.m) { tile = nt; take = true; }
-            }
-            if (take) {
-                tk.push_back(i);
-            } else {
-                df.push_back(i);
-                uint64_t nd = fits(op) ? op.nd : op.touch;
-                blockedNd |= nd;
-                blockedAll |= op.touch;
-            }
-        }
-        return tile;
-    };
+    std::vector<SchedRec> remaining(ops.size());
+    SchedScan sc{sp.m, 0};
+    bool untouching = false;               // an op on no qubit is never blocked
+    for (size_t i = 0; i < ops.size(); i++) {
+        const HOp& op = ops[i];
+        const bool fits = op.tileable && (unsigned)__builtin_popcountll(op.nd & ~lowMask) <= freeSlots;
+        remaining[i] = SchedRec{op.nd, op.touch, fits ? op.nd : op.touch, (int)i, fits};
+        sc.full |= op.touch;
+        untouching = untouching || op.touch == 0;
+    }
+    if (untouching || sc.full == 0) sc.full = ~0ULL;
     // the seeds of a list: the low qubits, then those plus the mixed qubits of
-    // each of its first fitting ops that reach above them
-    auto seedsOf = [&](const std::vector<int>& list, unsigned maxSeeds, std::vector<uint64_t>& out) {
+    // each of its first `maxSeeds` fitting ops that reach above them
+    auto seedsOf = [&](const std::vector<SchedRec>& list, unsigned maxSeeds, std::vector<uint64_t>& out) {
         out.assign(1, lowMask);
-        for (size_t r = 0; r < list.size() && out.size() <= maxSeeds; r++) {
-            const HOp& op = ops[list[r]];
-            if (fits(op) && (op.nd & ~lowMask) != 0) out.push_back(lowMask | op.nd);
+        unsigned found = 0;
+        for (size_t r = 0; r < list.size() && found < maxSeeds; r++) {
+            if (!list[r].fits || (list[r].nd & ~lowMask) == 0) continue;
+            found++;
+            const uint64_t seed = lowMask | list[r].nd;
+            if (std::find(out.begin(), out.end(), seed) == out.end()) out.push_back(seed);
         }
     };
-    std::vector<int> remaining(ops.size());
-    for (size_t i = 0; i < ops.size(); i++) remaining[i] = (int)i;
-    std::vector<int> tk, df, tk2, df2;
+    std::vector<SchedRec> tk, df;
     std::vector<uint64_t> s1, s2;
     while (!remaining.empty()) {
-        if (!fits(ops[remaining[0]])) {
+        if (!remaining[0].fits) {
             Stage st;
             st.tiled = false;
-            st.ops.push_back(remaining[0]);
+            st.ops.push_back(remaining[0].op);
             stages.push_back(st);
             remaining.erase(remaining.begin());
             continue;
@@ -197,15 +243,13 @@ std::vector<Stage> schedule(const std::vector<HOp>& ops, unsigned nq, SchedParam
         size_t bestScore = 0;
         seedsOf(remaining, seeds, s1);
         if (s1.size() > 1) {
+            const size_t n = std::min(window, remaining.size());
             for (size_t si = 0; si < s1.size(); si++) {
-                scan(remaining, window, s1[si], tk, df);
+                sc.split(remaining, n, s1[si], tk, df);
                 size_t score = tk.size(), best2 = 0;
                 if (look && !df.empty()) {
                     seedsOf(df, look, s2);
-                    for (uint64_t t2 : s2) {
-                        scan(df, window, t2, tk2, df2);
-                        best2 = std::max(best2, tk2.size());
-                    }
+                    for (uint64_t t2 : s2) best2 = std::max(best2, sc.count(df.data(), df.size(), t2, best2));
                 }
                 score += best2;
                 if (si == 0 || score > bestScore) {
@@ -214,14 +258,14 @@ std::vector<Stage> schedule(const std::vector<HOp>& ops, unsigned nq, SchedParam
                 }
             }
         }
-        std::vector<int> deferred;
         Stage st;
-        uint64_t tile = scan(remaining, remaining.size(), bestSeed, st.ops, deferred);
+        uint64_t tile = sc.split(remaining, remaining.size(), bestSeed, tk, df);
+        for (const SchedRec& r : tk) st.ops.push_back(r.op);
         for (unsigned q = 0; q < nq && (unsigned)__builtin_popcountll(tile) < sp.m; q++) tile |= 1ULL << q;
         for (unsigned q = 0; q < nq; q++) if ((tile >> q) & 1) st.tq.push_back(q);
         st.tiled = st.ops.size() > 1;
         stages.push_back(st);
-        remaining.swap(deferred);
+        remaining.swap(df);
     }
     if (const char* path = std::getenv("FSA_SCHEDULE_DUMP")) dump_schedule(path, ops, stages);
     return stages;
