@@ -482,6 +482,7 @@ __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi
         for (int b = 0; b < G; b++) if ((i >> b) & 1) base |= 1ULL << q[b];
         return base;
     };
+    touched(touch_lines<BLOCK>(ops, (size_t)numOps * sizeof(SweepOp)));
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t first = adjoint_block<R>() * (BLOCK / 64) + wave, step = (uint64_t)gridDim.x * (BLOCK / 64);
     for (uint64_t t = first; t < numTiles; t += step) {

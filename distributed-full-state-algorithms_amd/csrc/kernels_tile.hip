@@ -387,6 +387,12 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
             lmat[op.lmask + r * D + (c ^ (r & (D - 1)))] = M[(size_t)r * 2 * D + c];
         }
     };
+    // The items, before the first of them is read (a pass over a few tiles has
+    // nothing else to hide their latency: 150 items on one 12-qubit tile took
+    // 217 us and take 139).  Not in the MFMA kernels: it makes them spill
+    // (30-qubit passes 10.23 -> 10.54 ms).
+    uint32_t seen = 0;
+    if constexpr (VAR < 2) seen = touch_lines<TB>(items, (size_t)numItems * sizeof(TileOp));
     if constexpr (VAR == 2) {
         for (unsigned it = 0; it < numItems; it++) {
             const TileOp& op = items[it];
@@ -399,6 +405,7 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
 #pragma unroll
         for (int r = 0; r < ROWS; r++) s[((uint32_t)r << LOGTB) | tid] = mk<R>(bx[r], by[r]);
     }
+    if constexpr (VAR < 2) touched(seen);
     __syncthreads();
     uint64_t next = tile + gridDim.x;
     if (next < numTiles) FSA_PREFETCH(next);

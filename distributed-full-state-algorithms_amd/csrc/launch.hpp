@@ -25,6 +25,23 @@ __device__ __forceinline__ uint64_t stream_block() {
     return (uint64_t)(blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u;
 }
 
+// Reads one word of every 64 bytes of [p, p + bytes) with the whole workgroup,
+// all loads in flight at once, and returns a value to pass to touched() once
+// the loads have had their time.  Op lists are read through scalar loads, one
+// op at a time; from memory that no earlier kernel has brought into this XCD's
+// L2 each costs about a microsecond.
+template <int TB>
+__device__ __forceinline__ uint32_t touch_lines(const void* p, size_t bytes) {
+    const uint32_t* w = static_cast<const uint32_t*>(p);
+    uint32_t seen = 0;
+    for (size_t i = (size_t)threadIdx.x * 16; i < bytes / 4; i += TB * 16) seen ^= w[i];
+    return seen;
+}
+__device__ __forceinline__ void touched(uint32_t seen) {
+    const float f = __builtin_bit_cast(float, seen);
+    asm volatile("" : : "v"(f));         // an empty use: the loads stay
+}
+
 template <typename R> struct Offs32 { uint64_t o[32]; };
 
 // ---- streaming kernels: one HBM pass per operation ---------------------------
