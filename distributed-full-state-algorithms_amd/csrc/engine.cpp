@@ -922,8 +922,7 @@ void execute_impl(State& s, const std::vector<HOp>& ops, const std::vector<Stage
         // the tile leaves LDS, without an LDS round trip of their own.  An op
         // commutes with a later op when the later one mixes none of its qubits.
         std::vector<int> body, tail;
-        // (not in FP32 MFMA passes: their kernels have no registers left for it)
-        const bool drainDiag = env_flag("FSA_DRAIN_DIAG", true) && !(sizeof(R) == 4 && stageMfma);
+        const bool drainDiag = env_flag("FSA_DRAIN_DIAG", true);
         // one pass-end item holds a dephasing channel or up to two one-mask
         // diagonals (phase gadgets, Z-only Pauli gadgets and tensors)
         auto one_mask = [](const HOp& d) { return d.kind == OP_PHASE || (d.kind == OP_PAULI && d.mxy == 0); };
@@ -975,8 +974,7 @@ void execute_impl(State& s, const std::vector<HOp>& ops, const std::vector<Stage
             items.push_back(translate_diag4(ops[tail[0]], tail.size() > 1 ? &ops[tail[1]] : nullptr, pos, g.tileMask));
         flags[si] |= (tail.empty() ? 0u : 1u) << 8;
         count[si] = items.size() - first[si];
-        // every MFMA matrix of the pass goes to LDS (the left half of the real
-        // form, 2 * 4^k reals)
+        // every MFMA matrix of the pass goes to LDS (complex entries, 2 * 4^k reals)
         if (matsInLds) {
             uint32_t used = 0;
             for (size_t i = first[si]; i < items.size(); i++) {

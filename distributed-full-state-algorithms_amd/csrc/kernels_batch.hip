@@ -236,7 +236,7 @@ __device__ __forceinline__ void run_items(cx<R>* phi, uint32_t T, uint64_t base,
         bind_param(op, cs);
         // full tiles (T = ROWS * TB) load batches of four pairs before updating them
         // (one workgroup per CU: registers to spare)
-        tile_apply<R, TB, 1, 1, double, REV ? 2 * ROWS : ROWS, 4>(phi, REV ? 2 * T : T, base, op, mats);
+        tile_apply<R, TB, 1, double, REV ? 2 * ROWS : ROWS, 4>(phi, REV ? 2 * T : T, base, op, mats);
         __syncthreads();
     }
 }

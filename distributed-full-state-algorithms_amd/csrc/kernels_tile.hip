@@ -321,10 +321,8 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
     const uint32_t T = 1u << m;
     const uint32_t tid = threadIdx.x;
     const bool owner = tid < T;
-    // the last item (nDrain = 1) is an OP_DIAG4 applied at the write-back; FP32
-    // MFMA kernels (twice the accumulators per thread) have no registers for it
-    constexpr bool DRAIN = !(sizeof(R) == 4 && VAR >= 2);
-    const unsigned nDrain = DRAIN ? (flags >> 8) & 0xffu : 0u;
+    // the last item (nDrain = 1) is an OP_DIAG4 applied at the write-back
+    const unsigned nDrain = (flags >> 8) & 0xffu;
     // flags bit 6: the tiles are walked in bit-reversed index order, so the
     // tiles in flight at once differ in the highest qubits outside the tile
     // rather than the lowest (the HBM access pattern that measured faster).
@@ -364,33 +362,25 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
     R bx[ROWS], by[ROWS];
     uint64_t tile = blockIdx.x;
     if (tile >= numTiles) return;
-    // MFMA matrices go to LDS behind the tile, at their item's offset, in the
-    // order mat_lds_index reads them: the left half of the real form, or for
-    // the FP64 three-product form (tile_mfma3_form) U itself as complex
-    // entries.  VAR 2 copies every matrix of the pass once; VAR 3 (matrices
-    // beyond the LDS area) copies each one just before its item, at offset 0.
+    // MFMA matrices go to LDS behind the tile, at their item's offset, as the
+    // complex entries of U in mat_lds_index's order.  VAR 2 copies every matrix
+    // of the pass once; VAR 3 (matrices beyond the LDS area) copies each one
+    // just before its item, at offset 0.
     R* lmat = reinterpret_cast<R*>(smem_raw + ((size_t)sizeof(cx<R>) << m));
     auto stage_matrix = [&](const TileOp& op) {
         const uint32_t k = op.k, D = 1u << k;
-        const R* M = reinterpret_cast<const R*>(mats + op.mat_off);
-        if (tile_mfma3_form<R, TB>(k)) {
-            for (uint32_t e = tid; e < D * D; e += TB) {
-                const uint32_t r = e >> k, c = e & (D - 1);
-                R* dst = lmat + op.lmask + 2 * (r * D + (c ^ (r & (D - 1))));
-                dst[0] = M[(size_t)r * 2 * D + c];
-                dst[1] = M[(size_t)(r + D) * 2 * D + c];
-            }
-            return;
-        }
-        for (uint32_t e = tid; e < 2 * D * D; e += TB) {
+        const R* M = reinterpret_cast<const R*>(mats + op.mat_off);   // the real form, row-major
+        for (uint32_t e = tid; e < D * D; e += TB) {
             const uint32_t r = e >> k, c = e & (D - 1);
-            lmat[op.lmask + r * D + (c ^ (r & (D - 1)))] = M[(size_t)r * 2 * D + c];
+            R* dst = lmat + op.lmask + 2 * (r * D + (c ^ (r & (D - 1))));
+            dst[0] = M[(size_t)r * 2 * D + c];
+            dst[1] = M[(size_t)(r + D) * 2 * D + c];
         }
     };
     // The items, before the first of them is read (a pass over a few tiles has
     // nothing else to hide their latency: 150 items on one 12-qubit tile took
-    // 217 us and take 139).  Not in the MFMA kernels: it makes them spill
-    // (30-qubit passes 10.23 -> 10.54 ms).
+    // 217 us and take 139).  Not in the MFMA kernels, whose passes
+    // over many tiles it slows down (30 qubits: 9.34 -> 9.75 ms).
     uint32_t seen = 0;
     if constexpr (VAR < 2) seen = touch_lines<TB>(items, (size_t)numItems * sizeof(TileOp));
     if constexpr (VAR == 2) {
@@ -428,11 +418,14 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
                 }
             }
             // batched simple items, as many pairs per batch as the kernel has
-            // registers for (none in the MFMA kernels)
-            constexpr int GP = (TB != 512 || SW || VAR >= 2) ? 0
-                             : sizeof(R) == 4 ? (VAR == 0 ? 1 : 0)
+            // registers for.  In the MFMA kernels (and VAR 1 in FP32), against
+            // one at a time: 25-qubit FP32 passes 201 against 220 us, 30-qubit
+            // FP64 9.34 against 9.53 ms, 13-qubit density matrices 752 against
+            // 781 us.
+            constexpr int GP = (TB != 512 || SW) ? 0
+                             : sizeof(R) == 4 ? 1
                              : VAR == 0 ? 4 : 2;
-            tile_apply<R, TB, VAR, (ROWS >= 16 ? ROWS / 8 : 1), R, (GP ? ROWS : 0), GP>(s, T, base, op, mats, lmat);
+            tile_apply<R, TB, VAR, R, (GP ? ROWS : 0), GP>(s, T, base, op, mats, lmat);
             __syncthreads();
         }
         // The write-back of this tile and the loads of the tile after the next

@@ -161,10 +161,7 @@ __device__ __forceinline__ void tile_matk(cx<R>* s, uint32_t T, const TileOp& op
 // on 16x16x4 MFMA tiles.  Operand layout of v_mfma_*_16x16x4: lane l holds
 // A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator element j of lane l is
 // column l % 16, row 4 j + l / 16 for f64 and row 4 (l / 16) + j for f32
-// (measured on gfx950).  A wave task is one 16-row block
-// of the real matrix against four 16-group column blocks; the real matrix (in
-// the parameter buffer, row-major 2D x 2D) feeds A, the tile in LDS feeds B.
-// All inputs are read before the barrier, outputs written after it.
+// (measured on gfx950).  U feeds A, the tile in LDS feeds B.
 typedef double fsa_d4 __attribute__((ext_vector_type(4)));
 typedef float fsa_f4 __attribute__((ext_vector_type(4)));
 template <typename R> struct MfmaAcc;
@@ -181,14 +178,9 @@ template <> struct MfmaAcc<float> {
     }
 };
 
-// A tile of T amplitudes holds T / 512 wave tasks for every K (RB * groups / 64),
-// so each of the TB / 64 waves takes MAXT = T / (8 TB) of them: 1 for 4096
-// amplitudes at TB = 512, 2 for 8192.
-//
-// The A operand (the real matrix [[Ur, -Ui], [Ui, Ur]]) is read from LDS: M
-// holds its left half, the 2D x D reals [Ur; Ui], stored by mat_lds_index.
-// LDS reads keep the MFMA loops free of vector-memory loads, whose waits
-// would also wait for the next tile's prefetch (loads complete in order).
+// U is read from LDS too, stored by mat_lds_index: LDS reads keep the MFMA
+// loops free of vector-memory loads, whose waits would also wait for the next
+// tile's prefetch (loads complete in order).
 template <int D>
 __device__ __forceinline__ uint32_t mat_lds_index(uint32_t r, uint32_t c) {
     // columns XOR-swizzled by the row: the 16 rows a wave reads at one column
@@ -196,173 +188,121 @@ __device__ __forceinline__ uint32_t mat_lds_index(uint32_t r, uint32_t c) {
     return r * (uint32_t)D + (c ^ (r & (uint32_t)(D - 1)));
 }
 
-template <typename R, int K, int TB, int MAXT>
-__device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileOp& op, const R* __restrict__ M) {
+// M holds U as complex entries (mat_lds_index), so a lane gets ur and ui, and xr
+// and xi, in one LDS read each.  A wave owns 16-group column blocks with every
+// row of U: an amplitude is read once per sweep over the k-steps, and since no
+// other wave touches the groups of a block, the outputs are written without a
+// barrier between the waves.
+//   FP32, 4 or 5 targets: Yr and Yi apart, four products: 1 + RB LDS reads feed
+// 4 RB matrix operations.
+//   FP64, 4 targets: Gauss's three products P1 = Ur Xr, P2 = Ui Xi and
+// P3 = (Ur + Ui)(Xr + Xi) in one sweep; Yr = P1 - P2, Yi = P3 - (P1 + P2).
+//   FP64, 5 targets: P3 in a second sweep, added to -(P1 + P2): the 48
+// accumulator registers of one sweep over both row blocks make the kernel spill.
+//   3 targets: the 16 rows of one operation are Yr and Yi of the 8 outputs.
+// Bound by the matrix unit, whose operations (64 cycles in FP64, 32 in FP32)
+// hide the reads once two workgroups share a CU.  Tasks of one 16-row block
+// against four column blocks, with U and X read by halves, needed a workgroup
+// barrier, read an amplitude once per row block and left the kernels no
+// registers for batched simple items (tile_apply): with those, 25-qubit FP32
+// passes take 201 instead of 284 us, 30-qubit FP64 passes 9.34 instead of 10.24
+// ms, 13-qubit density-matrix passes 752 instead of 845 us.
+template <typename R, int K, int TB>
+__device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileOp& op, const cx<R>* __restrict__ M) {
     typedef typename MfmaAcc<R>::T acc_t;
-    constexpr int D = 1 << K, D2 = 2 * D;
-    constexpr int RB = D2 / 16;                 // 16-row blocks of the real matrix
+    constexpr int D = 1 << K;
+    constexpr int RB = D >= 16 ? D / 16 : 1;              // 16-row blocks of U
+    constexpr bool GAUSS = D >= 16 && sizeof(R) == 8;
+    constexpr bool TWICE = GAUSS && D == 32;
+    constexpr int PARTS = GAUSS && !TWICE ? 3 : D >= 16 ? 2 : 1;
     constexpr int WAVES = TB / 64;
+    // column blocks at once (16 to 32 accumulator registers in FP32, 16 to 32 in
+    // FP64); a full tile holds a multiple of NC * WAVES of them
+    constexpr int NC = sizeof(R) == 8 ? (D == 8 ? 2 : 1) : 32 / D;
+    static_assert(K >= 3 && K <= 5, "three to five targets");
     const uint32_t b0 = 1u << op.p[0], b1 = 1u << op.p[1], b2 = 1u << op.p[2];
     const uint32_t b3 = K > 3 ? 1u << op.p[3] : 0u;
     const uint32_t b4 = K > 4 ? 1u << op.p[4] : 0u;
     const uint32_t tm = b0 | b1 | b2 | b3 | b4;
-    const uint32_t groups = T >> K;
-    const uint32_t cb4 = groups / 64;          // groups of four 16-column blocks
-    const uint32_t tasks = RB * cb4;
+    const uint32_t blocks = T >> (K + 4);                 // column blocks of the tile
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t lr = lane & 15u, lk = lane >> 4;
-    acc_t acc[MAXT][4];
-    uint32_t taskId[MAXT];
-#pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        taskId[t] = wave + (uint32_t)t * WAVES;
-#pragma unroll
-        for (int c = 0; c < 4; c++) acc[t][c] = acc_t{0, 0, 0, 0};
-        if (taskId[t] >= tasks) continue;
-        const uint32_t rb = taskId[t] % RB, cbase = (taskId[t] / RB) * 4;
-        const uint32_t arow = rb * 16 + lr;                // real row of A this lane feeds
-        // B-fragment group bases of the four column blocks for this lane
-        uint32_t gb[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) gb[c] = ins0_mask32((cbase + (uint32_t)c) * 16 + lr, tm);
-        const R* sr = reinterpret_cast<const R*>(s);
-        auto kstep = [&](int ks, R a) {
-            const uint32_t r = (uint32_t)ks * 4 + lk;          // real row of X this lane feeds
-            const uint32_t off = mat_offset<K>(r & (D - 1), b0, b1, b2, b3, b4);
-            const uint32_t half = r < (uint32_t)D ? 0u : 1u;  // real or imaginary part only
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[t][c] = MfmaAcc<R>::step(a, sr[2 * (gb[c] | off) + half], acc[t][c]);
-        };
-        // not unrolled: four independent 64-cycle FP64 MFMAs per k-step cover
-        // the operand latency, and the loop stays clear of register spills.
-        // Columns C < D: A[row][C] = left[row][C]; columns C >= D:
-        // A[row][C] = -left[row + D][C - D] (row < D, the -Ui block) or
-        // left[row - D][C - D] (row >= D, the Ur block)
-        const uint32_t r2 = (arow + D) & (D2 - 1);
-        const R sgn = arow < (uint32_t)D ? (R)-1 : (R)1;
+    // the loops over column blocks and k-steps are not unrolled: the other waves
+    // of the SIMD cover the operand latency, and the kernels stay clear of spills
 #pragma unroll 1
-        for (int ks = 0; ks < D / 4; ks++) kstep(ks, M[mat_lds_index<D>(arow, (uint32_t)ks * 4 + lk)]);
-#pragma unroll 1
-        for (int ks = D / 4; ks < D2 / 4; ks++) kstep(ks, sgn * M[mat_lds_index<D>(r2, (uint32_t)ks * 4 + lk - D)]);
-    }
-    __syncthreads();
+    for (uint32_t cb = wave; cb < blocks; cb += NC * WAVES) {
+        acc_t acc[NC][RB][PARTS];
+        uint32_t gb[NC];
 #pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        if (taskId[t] >= tasks) continue;
-        const uint32_t rb = taskId[t] % RB, cbase = (taskId[t] / RB) * 4;
+        for (int c = 0; c < NC; c++) {
+            gb[c] = ins0_mask32((cb + (uint32_t)c * WAVES) * 16 + lr, tm);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint32_t gbc = ins0_mask32((cbase + (uint32_t)c) * 16 + lr, tm);
+            for (int b = 0; b < RB; b++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                // accumulator row j of this lane: FP64 4j + lane/16, FP32 4 (lane/16) + j
-                const uint32_t row = rb * 16 + (sizeof(R) == 8 ? 4u * (uint32_t)j + lk : lk * 4u + (uint32_t)j);
-                const uint32_t l = row & (D - 1);
-                R* dst = reinterpret_cast<R*>(&s[gbc | mat_offset<K>(l, b0, b1, b2, b3, b4)]);
-                dst[row < (uint32_t)D ? 0 : 1] = acc[t][c][j];
-            }
+                for (int h = 0; h < PARTS; h++) acc[c][b][h] = acc_t{0, 0, 0, 0};
         }
-    }
-}
-
-// FP64 gates of 4 or 5 targets in Gauss's three-product form (matrices in LDS,
-// 512-thread workgroups: tile_mfma3_form): a wave task is one 16-row block of U
-// (D / 16 of them) against two 16-group
-// column blocks.  A first sweep over the D / 4 k-steps accumulates P1 = Ur Xr
-// and P2 = Ui Xi, which become Yr = P1 - P2 and -(P1 + P2); a second sweep adds
-// P3 = (Ur + Ui)(Xr + Xi) to the latter, giving Yi.  Three quarters of the real
-// form's matrix operations, the same accumulator registers, and the same LDS
-// operand traffic (each sweep reads every amplitude once per row block of U,
-// as a 16-byte pair).  The tasks per tile are those of the real form (T / 512
-// for every K).  M holds U as complex entries, swizzled like the real form
-// (mat_lds_index), so that one 16-byte LDS read gives ur and ui.
-// The form is fixed at compile time: with the real form of these gates also
-// compiled in, the FP64 kernels exceed 128 VGPRs and spill; the 1024-thread
-// kernels spill with it and keep the real form.
-template <typename R, int TB>
-__host__ __device__ constexpr bool tile_mfma3_form(uint32_t k) {
-    return sizeof(R) == 8 && TB == 512 && (k == 4 || k == 5);
-}
-
-template <int K, int TB, int MAXT>
-__device__ __forceinline__ void tile_matk_mfma3(cx<double>* s, uint32_t T, const TileOp& op,
-                                                const cx<double>* __restrict__ M) {
-    typedef MfmaAcc<double>::T acc_t;
-    static_assert(K == 4 || K == 5, "three-product form: 16 or 32 rows of U");
-    constexpr int D = 1 << K;
-    constexpr int RB = D / 16;                  // 16-row blocks of U
-    constexpr int WAVES = TB / 64;
-    const uint32_t b0 = 1u << op.p[0], b1 = 1u << op.p[1], b2 = 1u << op.p[2], b3 = 1u << op.p[3];
-    const uint32_t b4 = K > 4 ? 1u << op.p[4] : 0u;
-    const uint32_t tm = b0 | b1 | b2 | b3 | b4;
-    const uint32_t groups = T >> K;
-    const uint32_t cb2 = groups / 32;          // pairs of 16-column blocks
-    const uint32_t tasks = RB * cb2;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t lr = lane & 15u, lk = lane >> 4;
-    acc_t yr[MAXT][2], yi[MAXT][2];
-    uint32_t taskId[MAXT];
-#pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        taskId[t] = wave + (uint32_t)t * WAVES;
-#pragma unroll
-        for (int c = 0; c < 2; c++) yr[t][c] = yi[t][c] = acc_t{0, 0, 0, 0};
-        if (taskId[t] >= tasks) continue;
-        const uint32_t rb = taskId[t] % RB, cbase = (taskId[t] / RB) * 2;
-        const uint32_t urow = rb * 16 + lr;               // row of U this lane feeds
-        uint32_t gb[2];
-#pragma unroll
-        for (int c = 0; c < 2; c++) gb[c] = ins0_mask32((cbase + (uint32_t)c) * 16 + lr, tm);
-        const cx<double>* mrow = M + urow * (uint32_t)D;
-        const uint32_t sw = urow & (uint32_t)(D - 1);
-        // not unrolled: the MFMAs of the other waves on the SIMD cover the
-        // operand latency, and the loops stay clear of register spills
 #pragma unroll 1
         for (uint32_t ks = 0; ks < (uint32_t)(D / 4); ks++) {
             const uint32_t col = ks * 4 + lk;             // column of U = row of X
-            const cx<double> u = mrow[col ^ sw];
             const uint32_t off = mat_offset<K>(col, b0, b1, b2, b3, b4);
+            cx<R> x[NC];
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const cx<double> x = s[gb[c] | off];
-                yr[t][c] = MfmaAcc<double>::step(u.x, x.x, yr[t][c]);
-                yi[t][c] = MfmaAcc<double>::step(u.y, x.y, yi[t][c]);
+            for (int c = 0; c < NC; c++) x[c] = s[gb[c] | off];
+#pragma unroll
+            for (int b = 0; b < RB; b++) {
+                const cx<R> u = M[mat_lds_index<D>(((uint32_t)b * 16 + lr) & (D - 1), col)];
+                // what multiplies xr and xi in this lane's row of the first accumulator
+                R ar = u.x, ai = -u.y;
+                if (PARTS == 1 && lr >= (uint32_t)D) { ar = u.y; ai = u.x; }
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    acc_t* y = acc[c][b];
+                    y[0] = MfmaAcc<R>::step(ar, x[c].x, y[0]);
+                    if constexpr (GAUSS) {
+                        y[1] = MfmaAcc<R>::step(u.y, x[c].y, y[1]);
+                        if constexpr (!TWICE) y[2] = MfmaAcc<R>::step(u.x + u.y, x[c].x + x[c].y, y[2]);
+                    } else {
+                        y[0] = MfmaAcc<R>::step(ai, x[c].y, y[0]);
+                        if constexpr (PARTS == 2) {
+                            y[1] = MfmaAcc<R>::step(u.y, x[c].x, y[1]);
+                            y[1] = MfmaAcc<R>::step(u.x, x[c].y, y[1]);
+                        }
+                    }
+                }
             }
         }
+        if constexpr (TWICE) {
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const acc_t p1 = yr[t][c], p2 = yi[t][c];
-            yr[t][c] = p1 - p2;
-            yi[t][c] = -(p1 + p2);
-        }
+            for (int b = 0; b < RB; b++) {
+                const acc_t p1 = acc[0][b][0], p2 = acc[0][b][1];
+                acc[0][b][0] = p1 - p2;
+                acc[0][b][1] = -(p1 + p2);
+            }
 #pragma unroll 1
-        for (uint32_t ks = 0; ks < (uint32_t)(D / 4); ks++) {
-            const uint32_t col = ks * 4 + lk;
-            const cx<double> u = mrow[col ^ sw];
-            const double us = u.x + u.y;
-            const uint32_t off = mat_offset<K>(col, b0, b1, b2, b3, b4);
+            for (uint32_t ks = 0; ks < (uint32_t)(D / 4); ks++) {
+                const uint32_t col = ks * 4 + lk;
+                const cx<R> x = s[gb[0] | mat_offset<K>(col, b0, b1, b2, b3, b4)];
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const cx<double> x = s[gb[c] | off];
-                yi[t][c] = MfmaAcc<double>::step(us, x.x + x.y, yi[t][c]);
+                for (int b = 0; b < RB; b++) {
+                    const cx<R> u = M[mat_lds_index<D>((uint32_t)b * 16 + lr, col)];
+                    acc[0][b][1] = MfmaAcc<R>::step(u.x + u.y, x.x + x.y, acc[0][b][1]);
+                }
             }
         }
-    }
-    __syncthreads();
 #pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        if (taskId[t] >= tasks) continue;
-        const uint32_t rb = taskId[t] % RB, cbase = (taskId[t] / RB) * 2;
+        for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const uint32_t gbc = ins0_mask32((cbase + (uint32_t)c) * 16 + lr, tm);
+            for (int b = 0; b < RB; b++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                // accumulator element j of this lane: row 4 j + lane / 16 of U
-                const uint32_t row = rb * 16 + 4u * (uint32_t)j + lk;
-                s[gbc | mat_offset<K>(row, b0, b1, b2, b3, b4)] = mk<double>(yr[t][c][j], yi[t][c][j]);
-            }
-        }
+                for (int j = 0; j < 4; j++) {
+                    // accumulator row j of this lane: FP64 4j + lane/16, FP32 4 (lane/16) + j
+                    const uint32_t row = (uint32_t)b * 16 + (sizeof(R) == 8 ? 4u * (uint32_t)j + lk : lk * 4u + (uint32_t)j);
+                    cx<R>* dst = &s[gb[c] | mat_offset<K>(row & (D - 1), b0, b1, b2, b3, b4)];
+                    const acc_t* y = acc[c][b];
+                    if constexpr (PARTS == 3) *dst = mk<R>(y[0][j] - y[1][j], y[2][j] - (y[0][j] + y[1][j]));
+                    else if constexpr (PARTS == 2) *dst = mk<R>(y[0][j], y[1][j]);
+                    else reinterpret_cast<R*>(dst)[row < (uint32_t)D ? 0 : 1] = y[0][j];
+                }
     }
 }
 
@@ -480,7 +420,7 @@ __device__ __forceinline__ void tile_quads(cx<R>* s, uint32_t n, uint32_t b0, ui
 // ROWS: amplitudes per thread of a full tile for the batched simple items; GP:
 // pairs per batch (singles 2 GP, density-matrix quartets GP / 2 in FP64; 0:
 // one at a time)
-template <typename R, int TB, int VAR, int MAXT = 1, typename C = R, int ROWS = 0, int GP = 0>
+template <typename R, int TB, int VAR, typename C = R, int ROWS = 0, int GP = 0>
 __device__ __forceinline__ void tile_apply(cx<R>* s, uint32_t T, uint64_t base, const TileOp& op,
                            const cx<C>* __restrict__ mats, const R* lmat = nullptr) {
     const uint32_t tid = threadIdx.x;
@@ -561,18 +501,10 @@ __device__ __forceinline__ void tile_apply(cx<R>* s, uint32_t T, uint64_t base, 
             if constexpr (VAR >= 2) {
                 static_assert(sizeof(C) == sizeof(R), "MFMA tiles compute in their storage precision");
                 // the matrix is in LDS: staged for the whole pass (VAR 2) or for this item (VAR 3)
-                const R* M = lmat + op.lmask;
-                if constexpr (tile_mfma3_form<R, TB>(4)) {
-                    if (op.k >= 4) {          // three-product form, complex U in LDS
-                        const cx<double>* Mc = reinterpret_cast<const cx<double>*>(M);
-                        if (op.k == 4) tile_matk_mfma3<4, TB, MAXT>(s, T, op, Mc);
-                        else tile_matk_mfma3<5, TB, MAXT>(s, T, op, Mc);
-                        return;
-                    }
-                }
-                if (op.k == 3) tile_matk_mfma<R, 3, TB, MAXT>(s, T, op, M);
-                else if (op.k == 4) tile_matk_mfma<R, 4, TB, MAXT>(s, T, op, M);
-                else tile_matk_mfma<R, 5, TB, MAXT>(s, T, op, M);
+                const cx<R>* M = reinterpret_cast<const cx<R>*>(lmat + op.lmask);
+                if (op.k == 3) tile_matk_mfma<R, 3, TB>(s, T, op, M);
+                else if (op.k == 4) tile_matk_mfma<R, 4, TB>(s, T, op, M);
+                else tile_matk_mfma<R, 5, TB>(s, T, op, M);
             }
             return;
         }
