@@ -83,7 +83,8 @@ bool has_mfma_gates(const std::vector<HOp>& ops) {
 SchedParams sched_params(unsigned nq, int precision, bool mfmaGates) {
     // FP32 tiles hold 2^13 amplitudes (64 KiB, two workgroups per CU) where
     // dense gates of 3-5 targets need them: their MFMA form works on full
-    // tiles.  Without such gates, 2^12 (32 KiB) lets four workgroups share a
+    // tiles, and 2^13 gives the fewer passes (160 gates on 25 qubits: 17 passes
+    // and 3590 us, against 20 and 3828 on 2^12).  Without such gates, 2^12 (32 KiB) lets four workgroups share a
     // CU, which hides more of each item's latency: the 24-qubit gadget
     // circuit's forward passes take 6.8 instead of 7.3 ms.
     const unsigned mmax = precision == FSA_FP64 ? (unsigned)tile_bits_max<double>()

@@ -421,7 +421,8 @@ __global__ __launch_bounds__(TB, (sizeof(R) == 8 && ROWS >= 16) ? 2 : 4) void k_
             // registers for.  In the MFMA kernels (and VAR 1 in FP32), against
             // one at a time: 25-qubit FP32 passes 201 against 220 us, 30-qubit
             // FP64 9.34 against 9.53 ms, 13-qubit density matrices 752 against
-            // 781 us.
+            // 781 us.  More pairs there change nothing (FP64 four, FP32 two: 9.47
+            // ms, 201 us) or spill (FP32 four: 908 us).
             constexpr int GP = (TB != 512 || SW) ? 0
                              : sizeof(R) == 4 ? 1
                              : VAR == 0 ? 4 : 2;
