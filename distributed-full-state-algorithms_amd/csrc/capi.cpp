@@ -147,23 +147,6 @@ void readback(State& s, double* dres, double* out, int n) {
     for (int i = 0; i < n; i++) out[i] = s.hres[i];
 }
 
-std::vector<PauliTermDev> dm_pauli_terms(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n) {
-    std::vector<PauliTermDev> terms(T);
-    for (unsigned t = 0; t < T; t++) {
-        uint64_t mxy = 0, myz = 0;
-        cd ph = 1.0;
-        for (unsigned q = 0; q < n; q++) {
-            unsigned c = paulis[(uint64_t)t * n + q];
-            if (c == 1 || c == 2) mxy |= 1ULL << q;
-            if (c == 2 || c == 3) myz |= 1ULL << q;
-            if (c == 2) ph *= cd(0, -1);
-        }
-        cd f = coeffs[t] * ph;
-        terms[t] = PauliTermDev{mxy, myz, f.real(), f.imag()};
-    }
-    return terms;
-}
-
 void create_state(unsigned N, bool dm, int prec, fsa_state** out) {
     need(out != nullptr, FSA_ERR_ARG, "null output handle");
     need(prec == FSA_FP64 || prec == FSA_FP32, FSA_ERR_ARG, "precision must be FSA_FP64 or FSA_FP32");
@@ -660,7 +643,7 @@ int fsa_densitymatrix_expecPauliString(fsa_state* h, const double* coeffs, unsig
         check_paulis(allPaulis, numTerms * s.N);
         flush(s);
         if (numTerms == 0) { out[0] = out[1] = 0; return; }
-        auto terms = dm_pauli_terms(coeffs, numTerms, allPaulis, s.N);
+        auto terms = pauli_terms(coeffs, numTerms, allPaulis, s.N, true);
         auto* dt = (const PauliTermDev*)s.ring.push(terms.data(), terms.size() * sizeof(PauliTermDev));
         double* ws = s.workspace(expec_workspace_doubles(s.N, numTerms) + 8);
         if (s.prec == FSA_FP64) launch_dm_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, dt, numTerms, ws + 8, ws);
@@ -750,12 +733,13 @@ int fsa_statevector_expecPauliSum(fsa_state* h, const double* coeffs, unsigned n
         check_paulis(paulis, numTerms * s.N);
         flush(s);
         if (numTerms == 0) { out[0] = out[1] = 0; return; }
-        PauliSum hs = pauli_sum(coeffs, numTerms, paulis, s.N);
-        push_pauli_sum(s.ring, hs);
-        const unsigned G = (unsigned)hs.groups.size();
-        double* ws = s.workspace(sv_expec_workspace_doubles(s.N, G) + 8);
-        if (s.prec == FSA_FP64) launch_sv_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, hs.dgroups, hs.dterms, G, ws + 8, ws);
-        else launch_sv_expec<float>(s.stream, (const cx<float>*)s.amps, s.N, hs.dgroups, hs.dterms, G, ws + 8, ws);
+        const PauliSumDev hs = push_pauli_sum(s.ring, coeffs, numTerms, paulis, s.N, s.prec, true);
+        double* ws = s.workspace(sv_expec_workspace_doubles(s.N, hs) + 8);
+        {
+            ProfScope prof(hs.groups ? "pauli_expec_groups" : "pauli_expec_terms", s.stream);
+            if (s.prec == FSA_FP64) launch_sv_expec<double>(s.stream, (const cx<double>*)s.amps, s.N, hs, ws + 8, ws);
+            else launch_sv_expec<float>(s.stream, (const cx<float>*)s.amps, s.N, hs, ws + 8, ws);
+        }
         hip_check(hipGetLastError(), "expec kernel");
         readback(s, ws, out, 2);
     });
@@ -772,11 +756,12 @@ int fsa_statevector_applyPauliSum(fsa_state* h, const double* coeffs, unsigned n
         flush(s);
         o.pending.clear();
         hip_check(hipStreamSynchronize(o.stream), "hipStreamSynchronize");
-        PauliSum hs = pauli_sum(coeffs, numTerms, paulis, s.N);
-        push_pauli_sum(s.ring, hs);
-        const unsigned G = (unsigned)hs.groups.size();
-        if (s.prec == FSA_FP64) launch_apply_pauli_sum<double>(s.stream, (const cx<double>*)s.amps, (cx<double>*)o.amps, s.N, hs.dgroups, hs.dterms, G);
-        else launch_apply_pauli_sum<float>(s.stream, (const cx<float>*)s.amps, (cx<float>*)o.amps, s.N, hs.dgroups, hs.dterms, G);
+        const PauliSumDev hs = push_pauli_sum(s.ring, coeffs, numTerms, paulis, s.N, s.prec, false);
+        {
+            ProfScope prof(hs.groups ? "pauli_apply_groups" : "pauli_apply_terms", s.stream);
+            if (s.prec == FSA_FP64) launch_apply_pauli_sum<double>(s.stream, (const cx<double>*)s.amps, (cx<double>*)o.amps, s.N, hs);
+            else launch_apply_pauli_sum<float>(s.stream, (const cx<float>*)s.amps, (cx<float>*)o.amps, s.N, hs);
+        }
         hip_check(hipGetLastError(), "apply Pauli sum");
         hip_check(hipStreamSynchronize(s.stream), "hipStreamSynchronize");
     });

@@ -17,7 +17,24 @@ using namespace fsa;
 
 namespace fsa {
 
-PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n) {
+std::vector<PauliTermDev> pauli_terms(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n, bool dm) {
+    std::vector<PauliTermDev> terms(T);
+    for (unsigned t = 0; t < T; t++) {
+        uint64_t mxy = 0, myz = 0;
+        cd ph = 1.0;
+        for (unsigned q = 0; q < n; q++) {
+            unsigned c = paulis[(uint64_t)t * n + q];
+            if (c == 1 || c == 2) mxy |= 1ULL << q;
+            if (c == 2 || c == 3) myz |= 1ULL << q;
+            if (c == 2) ph *= dm ? cd(0, -1) : cd(0, 1);
+        }
+        cd f = coeffs[t] * ph;
+        terms[t] = PauliTermDev{mxy, myz, f.real(), f.imag()};
+    }
+    return terms;
+}
+
+PauliGroups pauli_groups(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n) {
     struct Term { uint64_t mxy, myz; double c; uint32_t imag; };
     std::vector<Term> all(T);
     for (unsigned t = 0; t < T; t++) {
@@ -36,13 +53,13 @@ PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, uns
     std::stable_sort(all.begin(), all.end(), [](const Term& a, const Term& b) {
         return a.mxy != b.mxy ? a.mxy < b.mxy : a.imag < b.imag;
     });
-    PauliSum h;
-    h.terms.reserve(T);
+    PauliGroups h;
+    h.signs.reserve(T);
     for (unsigned t = 0; t < T; t++) {
         if (h.groups.empty() || h.groups.back().mxy != all[t].mxy || h.groups.back().imag != all[t].imag)
             h.groups.push_back(PauliGroupDev{all[t].mxy, t, t, all[t].imag, 0u});
         h.groups.back().t1 = t + 1;
-        h.terms.push_back(PauliSignDev{all[t].myz, all[t].c});
+        h.signs.push_back(PauliSignDev{all[t].myz, all[t].c});
     }
     for (size_t g = 0, first = 0; g < h.groups.size(); g++) {
         if ((h.groups[g].mxy ^ h.groups[first].mxy) >> PAULI_CHUNK_BITS) first = g;
@@ -51,15 +68,26 @@ PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, uns
     return h;
 }
 
-void push_pauli_sum(ParamRing& ring, PauliSum& h) {
+PauliSumDev push_pauli_sum(ParamRing& ring, const double* coeffs, unsigned T, const unsigned* paulis, unsigned n,
+                           int prec, bool expec) {
+    PauliSumDev d;
+    if (!pauli_sum_grouped(n, T, prec == FSA_FP64, expec)) {
+        const std::vector<PauliTermDev> terms = pauli_terms(coeffs, T, paulis, n, false);
+        d.terms = static_cast<const PauliTermDev*>(ring.push(terms.data(), T * sizeof(PauliTermDev)));
+        d.count = T;
+        return d;
+    }
+    const PauliGroups h = pauli_groups(coeffs, T, paulis, n);
     // one region: groups, then terms (both multiples of 8 bytes)
-    const size_t gb = h.groups.size() * sizeof(PauliGroupDev), tb = h.terms.size() * sizeof(PauliSignDev);
+    const size_t gb = h.groups.size() * sizeof(PauliGroupDev), tb = h.signs.size() * sizeof(PauliSignDev);
     std::vector<char> blob(gb + tb);
     std::memcpy(blob.data(), h.groups.data(), gb);
-    std::memcpy(blob.data() + gb, h.terms.data(), tb);
-    char* d = static_cast<char*>(ring.push(blob.data(), blob.size()));
-    h.dgroups = reinterpret_cast<const PauliGroupDev*>(d);
-    h.dterms = reinterpret_cast<const PauliSignDev*>(d + gb);
+    std::memcpy(blob.data() + gb, h.signs.data(), tb);
+    const char* p = static_cast<const char*>(ring.push(blob.data(), blob.size()));
+    d.groups = reinterpret_cast<const PauliGroupDev*>(p);
+    d.signs = reinterpret_cast<const PauliSignDev*>(p + gb);
+    d.count = (unsigned)h.groups.size();
+    return d;
 }
 
 HOp inverse(const HOp& op) {
@@ -503,11 +531,10 @@ void adjoint_impl(Circuit& c, State& psi0, const double* coeffs, unsigned T, con
     // the end instead of rescaling the states
     if (renorm) launch_norm2<R>(st, (const cx<R>*)phi.s.amps, phi.s.num(), ws, norms + 1);
 
-    PauliSum h = pauli_sum(coeffs, T, paulis, n);
-    push_pauli_sum(phi.s.ring, h);
+    const PauliSumDev h = push_pauli_sum(phi.s.ring, coeffs, T, paulis, n, psi0.prec, false);
     auto* a_phi = (cx<R>*)phi.s.amps;
     auto* a_lam = (cx<R>*)lam.s.amps;
-    launch_apply_pauli_sum<R>(st, a_phi, a_lam, n, h.dgroups, h.dterms, (unsigned)h.groups.size());
+    launch_apply_pauli_sum<R>(st, a_phi, a_lam, n, h);
 
     // Reverse sweep, op by op: for a gadget, <lambda|P_k|phi> and U_k^dag on phi
     // and on lambda in one pass over both states (k_adjoint_step); any other op

@@ -144,17 +144,19 @@ struct Circuit {
     std::shared_ptr<AdjointScratch> adj;
 };
 
-// A Pauli sum on n qubits (paulis[t * n + q], codes 0..3) in the grouped form
-// of launch_sv_expec and launch_apply_pauli_sum, groups in ascending X/Y mask
-// order and terms in the caller's order within a group.
-struct PauliSum {
+// The terms of a Pauli sum on n qubits (paulis[t * n + q], codes 0..3) with
+// coeff * (i or, for density matrices, -i)^{#Y}.
+std::vector<PauliTermDev> pauli_terms(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n, bool dm);
+// The same sum by groups: groups in ascending X/Y mask order, terms in the
+// caller's order within a group.
+struct PauliGroups {
     std::vector<PauliGroupDev> groups;
-    std::vector<PauliSignDev> terms;
-    const PauliGroupDev* dgroups = nullptr;   // set by push_pauli_sum
-    const PauliSignDev* dterms = nullptr;
+    std::vector<PauliSignDev> signs;
 };
-PauliSum pauli_sum(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n);
-void push_pauli_sum(ParamRing& ring, PauliSum& h);
+PauliGroups pauli_groups(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n);
+// a sum on a statevector in the form for its size (expec: <H>, else H psi), queued to the device
+PauliSumDev push_pauli_sum(ParamRing& ring, const double* coeffs, unsigned T, const unsigned* paulis, unsigned n,
+                           int prec, bool expec);
 
 // run ops on the state's stream; eager: each op as its own pass(es)
 void execute(State& s, const std::vector<HOp>& ops, const std::vector<Stage>& stages);

@@ -96,14 +96,16 @@ __global__ __launch_bounds__(BLOCK) void k_inner(const cx<R>* __restrict__ a, co
     if (threadIdx.x == 0) { part[2 * blockIdx.x] = vr; part[2 * blockIdx.x + 1] = vi; }
 }
 
-// Pauli-string sums of a density matrix.  Workgroup (t, c) handles term t over
-// chunk c of 2^N indices and writes f_t * (its partial sum)
-// (reference distributed_densitymatrix.hpp:322-344 / misc.hpp:16-38): only
-// entries with column c = r ^ mxy are nonzero, each sigma product equals
-// (-i)^{#Y} (-1)^{par(c & myz)}, so Tr(P rho) = (-i)^{#Y} sum_r (-1)^{..} rho[r + 2^N c].
+// Pauli-string sums.  Workgroup (t, c) handles term t over chunk c of 2^N (DM)
+// or 2^n (SV) indices and writes f_t * (its partial sum).
+//  DM (reference distributed_densitymatrix.hpp:322-344 / misc.hpp:16-38): only
+//  entries with column c = r ^ mxy are nonzero, each sigma product equals
+//  (-i)^{#Y} (-1)^{par(c & myz)}, so Tr(P rho) = (-i)^{#Y} sum_r (-1)^{..} rho[r + 2^N c].
+//  SV: <psi|P|psi> = i^{#Y} sum_j conj(psi_j) (-1)^{par(j1 & myz)} psi_{j1}, j1 = j ^ mxy;
+//  real, so the imaginary part is 0 (NaN where the real part is no number).
 constexpr uint64_t EXP_CHUNK = (uint64_t)BLOCK * 16;
 
-template <typename R>
+template <typename R, bool DM>
 __global__ __launch_bounds__(BLOCK) void k_pauli_expec(const cx<R>* __restrict__ a, unsigned nbits,
                                                        const PauliTermDev* __restrict__ terms,
                                                        unsigned chunks, double* __restrict__ part) {
@@ -116,14 +118,21 @@ __global__ __launch_bounds__(BLOCK) void k_pauli_expec(const cx<R>* __restrict__
     for (uint64_t r = start + threadIdx.x; r < end; r += BLOCK) {
         uint64_t r1 = r ^ term.mxy;
         double sg = par64(r1 & term.myz) ? -1.0 : 1.0;
-        cx<R> v = a[r + (r1 << nbits)];
-        vr += sg * (double)v.x;
-        vi += sg * (double)v.y;
+        if (DM) {
+            cx<R> v = a[r + (r1 << nbits)];
+            vr += sg * (double)v.x;
+            vi += sg * (double)v.y;
+        } else {
+            cx<R> x = a[r], y = a[r1];
+            vr += sg * ((double)x.x * (double)y.x + (double)x.y * (double)y.y);
+            vi += sg * ((double)x.x * (double)y.y - (double)x.y * (double)y.x);
+        }
     }
     block_sum2(vr, vi);
     if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = term.fr * vr - term.fi * vi;
-        part[2 * blockIdx.x + 1] = term.fr * vi + term.fi * vr;
+        const double re = term.fr * vr - term.fi * vi;
+        part[2 * blockIdx.x] = re;
+        part[2 * blockIdx.x + 1] = DM ? term.fr * vi + term.fi * vr : re - re;
     }
 }
 
@@ -578,17 +587,35 @@ __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi
     }
 }
 
+// out[j] = sum_t f_t (-1)^{par(j1 & myz_t)} in[j1], j1 = j ^ mxy_t
+template <typename R>
+__global__ __launch_bounds__(BLOCK) void k_apply_pauli_terms(const cx<R>* __restrict__ in, cx<R>* __restrict__ out,
+                                                             uint64_t num, const PauliTermDev* __restrict__ terms,
+                                                             unsigned numTerms) {
+    const uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (j >= num) return;
+    double ar = 0, ai = 0;
+    for (unsigned t = 0; t < numTerms; t++) {
+        const PauliTermDev term = terms[t];
+        uint64_t j1 = j ^ term.mxy;
+        double sg = par64(j1 & term.myz) ? -1.0 : 1.0;
+        cx<R> v = in[j1];
+        double fr = sg * term.fr, fi = sg * term.fi;
+        ar += fr * (double)v.x - fi * (double)v.y;
+        ai += fr * (double)v.y + fi * (double)v.x;
+    }
+    out[j] = mk<R>((R)ar, (R)ai);
+}
+
 // A Pauli sum H on a statevector, grouped by X/Y mask (PauliGroupDev): either
 // <psi|H|psi> (EXPEC, one partial per workgroup) or out = H psi.  A thread owns
 // ITEMS amplitudes j = chunk base + 256 i + tid and walks the groups: it takes
 // psi_{j ^ mxy} once per group, sums the group's coefficients with their signs,
 // and multiplies once.  Signs split into a part fixed for the workgroup, a part
 // of the lane and a part of i, so a term costs one lane parity however many
-// amplitudes a thread owns.
-//   WIDE (2^20 amplitudes and more): ITEMS = 8, chunks of 2^PAULI_CHUNK_BITS.
-// Groups that agree above the chunk read the same other chunk, which goes to
-// LDS once for all of them; a group that is alone there is loaded straight
-// into registers.  Otherwise ITEMS = 1, eight groups' loads in flight.
+// amplitudes a thread owns.  Groups that agree above the chunk read the same
+// other chunk, which goes to LDS once for all of them; a group that is alone
+// there is loaded straight into registers.
 //   EXPEC keeps psi_j in registers for all groups.  A Pauli string with a real
 // coefficient is Hermitian, so the pair (j, j ^ mxy) contributes twice the real
 // part of one of its two products: groups whose top X/Y qubit lies above the
@@ -599,32 +626,22 @@ __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi
 // weight 1-4: <H> 6.19 -> 0.65 ms, H psi 1.82 -> 1.12 ms against one pass per
 // term (which left 409600 partials to one workgroup); without the LDS copy of
 // shared chunks 0.82 and 1.45 ms.
-template <typename R, bool WIDE, bool EXPEC>
+template <typename R, bool EXPEC>
 __global__ __launch_bounds__(BLOCK) void k_pauli_groups(const cx<R>* __restrict__ a, cx<R>* __restrict__ out,
                                                         uint64_t num, const PauliGroupDev* __restrict__ groups,
                                                         const PauliSignDev* __restrict__ terms, unsigned numGroups,
-                                                        unsigned splits, double* __restrict__ part) {
-    constexpr int ITEMS = WIDE ? 8 : 1, GB = WIDE ? 1 : 8;
-    constexpr uint64_t CHUNK = (uint64_t)BLOCK * ITEMS;
-    static_assert(!WIDE || CHUNK == 1ULL << PAULI_CHUNK_BITS, "group runs are built for this chunk");
-    __shared__ cx<R> other[WIDE ? CHUNK : 1];
+                                                        double* __restrict__ part) {
+    constexpr uint64_t CHUNK = 1ULL << PAULI_CHUNK_BITS;
+    constexpr int ITEMS = (int)(CHUNK / BLOCK);
+    __shared__ cx<R> other[CHUNK];
     const uint32_t tid = threadIdx.x;
-    const bool valid = tid < num;               // states of fewer than 256 amplitudes
-    const uint32_t lanes = num < BLOCK ? (uint32_t)num - 1u : BLOCK - 1u;
-    // workgroup b takes every (gridDim / splits)-th chunk and the b % splits-th share of the groups
-    const unsigned split = blockIdx.x % splits, stride = gridDim.x / splits;
-    const unsigned perSplit = (numGroups + splits - 1) / splits;
-    const unsigned gFirst = split * perSplit;
-    const unsigned gLast = gFirst + perSplit < numGroups ? gFirst + perSplit : numGroups;
-    const uint64_t numChunks = (num + CHUNK - 1) / CHUNK;
     double v = 0;
-    for (uint64_t chunk = blockIdx.x / splits; chunk < numChunks; chunk += stride) {
-        const uint64_t base = chunk * CHUNK;
+    for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < num; base += (uint64_t)gridDim.x * CHUNK) {
         cx<R> x[ITEMS];
         double ar[ITEMS], ai[ITEMS];
 #pragma unroll
         for (int i = 0; i < ITEMS; i++) {
-            if constexpr (EXPEC) x[i] = a[base + (uint32_t)i * BLOCK + (tid & lanes)];
+            if constexpr (EXPEC) x[i] = a[base + (uint32_t)i * BLOCK + tid];
             else ar[i] = ai[i] = 0;
         }
         // amplitude of item i under group gr is element ((i ^ mi) * BLOCK + (tid ^ mxy)) of chunk base ^ mxy
@@ -650,64 +667,49 @@ __global__ __launch_bounds__(BLOCK) void k_pauli_groups(const cx<R>* __restrict_
                 if constexpr (EXPEC) {
                     // Re(conj(x) y) for a real factor, Re(i conj(x) y) for an imaginary one
                     const double xx = (double)x[i].x, xy = (double)x[i].y;
-                    const double w = gr.imag ? xy * yx - xx * yy : xx * yx + xy * yy;
-                    if (valid) v += weight * c[i] * w;
+                    v += weight * c[i] * (gr.imag ? xy * yx - xx * yy : xx * yx + xy * yy);
                 } else {
                     ar[i] += gr.imag ? -c[i] * yy : c[i] * yx;
                     ai[i] += gr.imag ? c[i] * yx : c[i] * yy;
                 }
             }
         };
-        if constexpr (WIDE) {
-            for (unsigned g = 0; g < numGroups;) {
-                const PauliGroupDev gr = groups[g];
-                const unsigned run = gr.run;
-                double weight = 1.0;
-                if (EXPEC && gr.mxy >= CHUNK) {      // the pairs' other halves are in another chunk
-                    weight = 2.0;
-                    if ((base >> (63 - __builtin_clzll(gr.mxy))) & 1ULL) { g += run; continue; }
-                }
-                const cx<R>* src = a + (base ^ (gr.mxy & ~(CHUNK - 1)));
-                cx<R> y[ITEMS];
-                if (run == 1) {
-                    const uint32_t mi = item_mask(gr.mxy), l = (tid ^ (uint32_t)gr.mxy) & (BLOCK - 1u);
-#pragma unroll
-                    for (int i = 0; i < ITEMS; i++) y[i] = src[((uint32_t)i ^ mi) * BLOCK + l];
-                    add_group(gr, y, weight);
-                    g++;
-                    continue;
-                }
-#pragma unroll
-                for (int i = 0; i < ITEMS; i++) y[i] = src[(uint32_t)i * BLOCK + tid];
-                __syncthreads();                     // the previous run has been read
-#pragma unroll
-                for (int i = 0; i < ITEMS; i++) other[(uint32_t)i * BLOCK + tid] = y[i];
-                __syncthreads();
-                for (const unsigned end = g + run; g < end; g++) {
-                    const PauliGroupDev gi = groups[g];
-                    const uint32_t mi = item_mask(gi.mxy), l = (tid ^ (uint32_t)gi.mxy) & (BLOCK - 1u);
-#pragma unroll
-                    for (int i = 0; i < ITEMS; i++) y[i] = other[((uint32_t)i ^ mi) * BLOCK + l];
-                    add_group(gi, y, weight);
-                }
+        for (unsigned g = 0; g < numGroups;) {
+            const PauliGroupDev gr = groups[g];
+            const unsigned run = gr.run;
+            double weight = 1.0;
+            if (EXPEC && gr.mxy >= CHUNK) {      // the pairs' other halves are in another chunk
+                weight = 2.0;
+                if ((base >> (63 - __builtin_clzll(gr.mxy))) & 1ULL) { g += run; continue; }
             }
-        } else {
-            for (unsigned g = gFirst; g < gLast; g += GB) {
-                cx<R> y[GB][ITEMS];
+            const cx<R>* src = a + (base ^ (gr.mxy & ~(CHUNK - 1)));
+            cx<R> y[ITEMS];
+            if (run == 1) {
+                const uint32_t mi = item_mask(gr.mxy), l = (tid ^ (uint32_t)gr.mxy) & (BLOCK - 1u);
 #pragma unroll
-                for (int q = 0; q < GB; q++) {
-                    const uint64_t m = groups[g + q < gLast ? g + q : gLast - 1].mxy;
-                    y[q][0] = a[(base ^ (m & ~(CHUNK - 1))) + ((tid ^ (uint32_t)m) & lanes)];
-                }
+                for (int i = 0; i < ITEMS; i++) y[i] = src[((uint32_t)i ^ mi) * BLOCK + l];
+                add_group(gr, y, weight);
+                g++;
+                continue;
+            }
 #pragma unroll
-                for (int q = 0; q < GB; q++)
-                    if (g + q < gLast) add_group(groups[g + q], y[q], 1.0);
+            for (int i = 0; i < ITEMS; i++) y[i] = src[(uint32_t)i * BLOCK + tid];
+            __syncthreads();                     // the previous run has been read
+#pragma unroll
+            for (int i = 0; i < ITEMS; i++) other[(uint32_t)i * BLOCK + tid] = y[i];
+            __syncthreads();
+            for (const unsigned end = g + run; g < end; g++) {
+                const PauliGroupDev gi = groups[g];
+                const uint32_t mi = item_mask(gi.mxy), l = (tid ^ (uint32_t)gi.mxy) & (BLOCK - 1u);
+#pragma unroll
+                for (int i = 0; i < ITEMS; i++) y[i] = other[((uint32_t)i ^ mi) * BLOCK + l];
+                add_group(gi, y, weight);
             }
         }
         if constexpr (!EXPEC) {
 #pragma unroll
             for (int i = 0; i < ITEMS; i++)
-                if (valid) out[base + (uint32_t)i * BLOCK + tid] = mk<R>((R)ar[i], (R)ai[i]);
+                out[base + (uint32_t)i * BLOCK + tid] = mk<R>((R)ar[i], (R)ai[i]);
         }
     }
     if constexpr (EXPEC) {
@@ -906,13 +908,19 @@ unsigned launch_sweep(hipStream_t s, bool rev, cx<R>* phi, cx<R>* lam, unsigned 
 }
 
 // ws must hold 2 * numTerms * ceil(2^nbits / EXP_CHUNK) doubles
+template <typename R, bool DM>
+static void launch_expec_terms(hipStream_t s, const cx<R>* a, unsigned nbits, const PauliTermDev* dterms,
+                               unsigned numTerms, double* ws, double* dout) {
+    unsigned chunks = (unsigned)(((1ULL << nbits) + EXP_CHUNK - 1) / EXP_CHUNK);
+    unsigned nb = numTerms * chunks;
+    hipLaunchKernelGGL((k_pauli_expec<R, DM>), dim3(nb), dim3(BLOCK), 0, s, a, nbits, dterms, chunks, ws);
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(BLOCK), 0, s, ws, nb, dout);
+}
+
 template <typename R>
 void launch_dm_expec(hipStream_t s, const cx<R>* rho, unsigned N, const PauliTermDev* dterms,
                      unsigned numTerms, double* ws, double* dout) {
-    unsigned chunks = (unsigned)(((1ULL << N) + EXP_CHUNK - 1) / EXP_CHUNK);
-    unsigned nb = numTerms * chunks;
-    hipLaunchKernelGGL(k_pauli_expec<R>, dim3(nb), dim3(BLOCK), 0, s, rho, N, dterms, chunks, ws);
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(BLOCK), 0, s, ws, nb, dout);
+    launch_expec_terms<R, true>(s, rho, N, dterms, numTerms, ws, dout);
 }
 
 uint64_t expec_workspace_doubles(unsigned nbits, unsigned numTerms) {
@@ -921,51 +929,39 @@ uint64_t expec_workspace_doubles(unsigned nbits, unsigned numTerms) {
 
 namespace {
 
-// Form of a grouped Pauli sum: eight amplitudes per thread once that still
-// leaves PAULI_WIDE_MIN / 2048 = 512 workgroups; smaller states have one amplitude per
-// thread and eight groups in flight instead, and <H> splits its groups over
-// workgroups until there are about 1024.
-constexpr uint64_t PAULI_WIDE_MIN = 1ULL << 20;
-constexpr unsigned PAULI_MAX_BLOCKS = 4096;
-
-struct PauliForm { bool wide; unsigned blocks, splits; };
-
-PauliForm pauli_form(unsigned n, unsigned numGroups, bool expec) {
-    const uint64_t num = 1ULL << n;
-    PauliForm f;
-    f.wide = num >= PAULI_WIDE_MIN;
-    const uint64_t chunk = (uint64_t)BLOCK * (f.wide ? 8 : 1);
-    f.blocks = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((num + chunk - 1) / chunk, PAULI_MAX_BLOCKS));
-    f.splits = 1;
-    if (expec && !f.wide)
-        f.splits = std::max(1u, std::min((numGroups + 7) / 8, 1024u / std::min(f.blocks, 1024u)));
-    f.blocks *= f.splits;
-    return f;
+// workgroups of k_pauli_groups: H psi takes a chunk each, <H> leaves few partials
+unsigned pauli_group_blocks(unsigned n, bool expec) {
+    const uint64_t chunks = 1ULL << (n - PAULI_CHUNK_BITS);
+    return (unsigned)(expec ? std::min<uint64_t>(chunks, 4096) : chunks);
 }
 
 }  // namespace
 
-uint64_t sv_expec_workspace_doubles(unsigned n, unsigned numGroups) {
-    return 2ULL * pauli_form(n, numGroups, true).blocks;
+uint64_t sv_expec_workspace_doubles(unsigned n, const PauliSumDev& h) {
+    return h.groups ? 2ULL * pauli_group_blocks(n, true) : expec_workspace_doubles(n, h.count);
 }
 
 template <typename R>
-void launch_sv_expec(hipStream_t s, const cx<R>* psi, unsigned n, const PauliGroupDev* dgroups,
-                     const PauliSignDev* dterms, unsigned numGroups, double* ws, double* dout) {
-    const PauliForm f = pauli_form(n, numGroups, true);
-    auto* kern = f.wide ? k_pauli_groups<R, true, true> : k_pauli_groups<R, false, true>;
-    hipLaunchKernelGGL(kern, dim3(f.blocks), dim3(BLOCK), 0, s, psi, (cx<R>*)nullptr, (uint64_t)(1ULL << n), dgroups,
-                       dterms, numGroups, f.splits, ws);
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(BLOCK), 0, s, ws, f.blocks, dout);
+void launch_sv_expec(hipStream_t s, const cx<R>* psi, unsigned n, const PauliSumDev& h, double* ws, double* dout) {
+    if (!h.groups) {
+        launch_expec_terms<R, false>(s, psi, n, h.terms, h.count, ws, dout);
+        return;
+    }
+    const unsigned nb = pauli_group_blocks(n, true);
+    hipLaunchKernelGGL((k_pauli_groups<R, true>), dim3(nb), dim3(BLOCK), 0, s, psi, (cx<R>*)nullptr,
+                       (uint64_t)(1ULL << n), h.groups, h.signs, h.count, ws);
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(BLOCK), 0, s, ws, nb, dout);
 }
 
 template <typename R>
-void launch_apply_pauli_sum(hipStream_t s, const cx<R>* in, cx<R>* out, unsigned n, const PauliGroupDev* dgroups,
-                            const PauliSignDev* dterms, unsigned numGroups) {
-    const PauliForm f = pauli_form(n, numGroups, false);
-    auto* kern = f.wide ? k_pauli_groups<R, true, false> : k_pauli_groups<R, false, false>;
-    hipLaunchKernelGGL(kern, dim3(f.blocks), dim3(BLOCK), 0, s, in, out, (uint64_t)(1ULL << n), dgroups, dterms,
-                       numGroups, f.splits, (double*)nullptr);
+void launch_apply_pauli_sum(hipStream_t s, const cx<R>* in, cx<R>* out, unsigned n, const PauliSumDev& h) {
+    const uint64_t num = 1ULL << n;
+    if (!h.groups)
+        hipLaunchKernelGGL(k_apply_pauli_terms<R>, dim3((unsigned)((num + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, s, in,
+                           out, num, h.terms, h.count);
+    else
+        hipLaunchKernelGGL((k_pauli_groups<R, false>), dim3(pauli_group_blocks(n, false)), dim3(BLOCK), 0, s, in, out,
+                           num, h.groups, h.signs, h.count, (double*)nullptr);
 }
 
 template <typename R>
@@ -1025,10 +1021,8 @@ void launch_f32_to_f64(hipStream_t s, const cx<float>* in, cx<double>* out, uint
                                              double*, uint64_t, const AdjointDiagDev*);                         \
     template void launch_dm_expec<R>(hipStream_t, const cx<R>*, unsigned, const PauliTermDev*, unsigned,       \
                                      double*, double*);                                                       \
-    template void launch_sv_expec<R>(hipStream_t, const cx<R>*, unsigned, const PauliGroupDev*,                \
-                                     const PauliSignDev*, unsigned, double*, double*);                        \
-    template void launch_apply_pauli_sum<R>(hipStream_t, const cx<R>*, cx<R>*, unsigned, const PauliGroupDev*, \
-                                            const PauliSignDev*, unsigned);                                   \
+    template void launch_sv_expec<R>(hipStream_t, const cx<R>*, unsigned, const PauliSumDev&, double*, double*); \
+    template void launch_apply_pauli_sum<R>(hipStream_t, const cx<R>*, cx<R>*, unsigned, const PauliSumDev&);  \
     template void launch_partial_trace<R>(hipStream_t, const cx<R>*, cx<R>*, unsigned, const unsigned*,       \
                                           unsigned);                                                          \
     template void launch_init_gaussian<R>(hipStream_t, cx<R>*, unsigned, uint64_t);                           \
