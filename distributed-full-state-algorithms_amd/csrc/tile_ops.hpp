@@ -69,12 +69,18 @@ __device__ __forceinline__ void tile_matk(cx<R>* s, uint32_t T, const TileOp& op
     constexpr int OUTMAX = sizeof(C) == 8 ? 8 : 16;
     constexpr int OUT = D < OUTMAX ? D : OUTMAX;
     // whole groups per thread, written in place; a full tile has >= TB groups only when D <= OUT
-    if constexpr (D <= 8) if (groups >= (uint32_t)TB) {
+    constexpr bool BY_ROWS = D <= 4 || (D == 8 && sizeof(C) == 8);
+    if constexpr (BY_ROWS) if (groups >= (uint32_t)TB) {
         // The inputs of a group are read together, then its outputs are formed
         // row by row: one LDS wait per group, and a row of the matrix is
         // contiguous, so its scalar loads are wide and run ahead by rows.
         // (Column by column, with one input and one matrix column at a time,
-        // every input cost an LDS wait and a scalar wait.)
+        // every input cost an LDS wait and a scalar wait.)  Not for three
+        // targets in FP32, whose larger tiles take the MFMA form: on the one
+        // tile that is left, 12 qubits, no earlier tile has brought the matrix
+        // into the caches, and its eight lines arrive one row after another
+        // where the first column asks for all of them (40 gates: 187 against
+        // 158 us).
         for (uint32_t g = tid; g < groups; g += TB) {
             const uint32_t b = ins0_mask32(g, tm);
             cx<C> x[D];
@@ -90,7 +96,7 @@ __device__ __forceinline__ void tile_matk(cx<R>* s, uint32_t T, const TileOp& op
         }
         return;
     }
-    if constexpr (D > 8 && D <= OUT) if (groups >= (uint32_t)TB) {
+    if constexpr (!BY_ROWS && D <= OUT) if (groups >= (uint32_t)TB) {
         for (uint32_t g = tid; g < groups; g += TB) {
             const cx<C>* m = mat;
             const uint32_t b = ins0_mask32(g, tm);
