@@ -158,13 +158,13 @@ struct BlobBuilder {
                     t.p[0] = ngrad++;
                     t.mat_off = numJobs + (uint32_t)op.param;
                     t.param = NO_PARAM;
-                    // the gadget's inverse right after it: one fused sweep (item field k = 1)
-                    if (ii + 1 < s.ops.size()) {
-                        const int ni = s.ops[ii + 1];
-                        const HOp& nx = ops[ni];
-                        if ((nx.kind == OP_PAULI || nx.kind == OP_PHASE) && nx.param == op.param && sign[ni] < 0)
-                            t.k = 1;
-                    }
+                    // The kernel sums the term while it applies the gadget's inverse: that
+                    // must be the next op of the pass.  It is: the two have the same masks
+                    // and are neighbours, so the scheduler takes both or neither.
+                    const int ni = ii + 1 < s.ops.size() ? s.ops[ii + 1] : -1;
+                    need(ni >= 0 && (ops[ni].kind == OP_PAULI || ops[ni].kind == OP_PHASE) &&
+                             ops[ni].param == op.param && sign[ni] < 0,
+                         FSA_ERR_INTERNAL, "a gradient item is not followed by its gadget's inverse");
                 } else if (op.param >= 0 && (op.kind == OP_PAULI || op.kind == OP_PHASE)) {
                     t.param = (uint32_t)op.param;
                     t.f[4] = op.pw.real();

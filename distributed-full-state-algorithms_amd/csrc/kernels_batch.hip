@@ -75,26 +75,11 @@ __device__ __forceinline__ void bind_param(TileOp& op, const double* __restrict_
     }
 }
 
-// Im <lambda|P|phi> over one tile: sum_l conj(lam_l) i^#Y (-1)^{par(k & myz)} phi_k, k = l ^ mxy
-template <typename R, int TB>
-__device__ __forceinline__ double grad_partial(const cx<R>* phi, const cx<R>* lam, uint32_t T, uint64_t base,
-                                               const TileOp& op) {
-    const uint32_t bp = par64(base & op.gmask);
-    double ar = 0, ai = 0;
-    for (uint32_t l = threadIdx.x; l < T; l += TB) {
-        const uint32_t k = l ^ op.lmask;
-        const cx<R> x = lam[l], y = phi[k];
-        const double sg = (bp ^ par32(k & op.lmask2)) ? -1.0 : 1.0;
-        ar += sg * ((double)x.x * (double)y.x + (double)x.y * (double)y.y);
-        ai += sg * ((double)x.x * (double)y.y - (double)x.y * (double)y.x);
-    }
-    return op.f[0] * ai + op.f[1] * ar;
-}
-
-// A gradient item fused with the inverse gadget after it (same Pauli masks):
-// one sweep over the pairs (l, l ^ mxy) of both tiles accumulates the item's
-// Im <lambda|P|phi> terms (as grad_partial) and applies the gadget `o` to phi
-// and lambda with the arithmetic of tile_apply's OP_PAULI / OP_PHASE.  ROWS:
+// A gradient item and the inverse gadget after it (same Pauli masks): one sweep
+// over the pairs (l, l ^ mxy) of both tiles accumulates Im <lambda|P|phi> =
+// Im sum_l conj(lam_l) i^#Y (-1)^{par(k & myz)} phi_k, k = l ^ mxy, and applies
+// the gadget `o` to phi and lambda with the arithmetic of tile_apply's
+// OP_PAULI / OP_PHASE.  ROWS:
 // amplitudes per thread of a full tile, whose loads are then issued together.
 template <typename R, int TB, int ROWS>
 __device__ __forceinline__ double grad_apply(cx<R>* phi, cx<R>* lam, uint32_t T, uint64_t base, const TileOp& g,
@@ -215,22 +200,14 @@ __device__ __forceinline__ void run_items(cx<R>* phi, uint32_t T, uint64_t base,
     for (uint32_t i = i0; i < i0 + ni; i++) {
         TileOp op = items[i];
         if (REV && op.kind == OP_GRAD) {
-            double v;
-            const bool fused = op.k == 1u;  // the next item is this gadget's inverse
-            if (fused) {
-                TileOp inv = items[i + 1];
-                bind_param(inv, cs);
-                v = grad_apply<R, TB, ROWS>(phi, lam, T, base, op, inv);
-                i++;
-            } else {
-                v = grad_partial<R, TB>(phi, lam, T, base, op);
-            }
-            v = bwave_sum(v);
+            TileOp inv = items[++i];        // the planner puts the gadget's inverse next to it
+            bind_param(inv, cs);
+            const double v = bwave_sum(grad_apply<R, TB, ROWS>(phi, lam, T, base, op, inv));
             if ((threadIdx.x & 63u) == 0) {
                 double* r = gacc + (threadIdx.x >> 6) * BATCH_STAGE_GRADS + op.p[0];
                 *r = firstTile ? v : *r + v;
             }
-            if (fused) __syncthreads();     // the tiles were written (a gradient sum alone only reads them)
+            __syncthreads();
             continue;
         }
         bind_param(op, cs);
@@ -374,7 +351,7 @@ __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs,
             for (uint64_t t = 0; t < numTiles; t++) {
                 const uint64_t base = pdep64(t, outMask);
                 run_items<R, TB, REV, KMAX>(lds, T, base, items, st.item0, st.nitems, mats, cs, gacc, t == 0);
-                __syncthreads();   // the last item may be a gradient sum still reading other rows
+                __syncthreads();   // tile t is final in LDS
                 // Each thread writes its own rows of tile t back and fills them
                 // with tile t + 1; the wait makes tile t + 1's loads land before the
                 // first store of tile t is issued (vector memory operations

@@ -1,0 +1,21 @@
+"""Conditions that the host planners guarantee to the kernels, on the CPU.
+
+The batch kernel sums a gradient term in the sweep that applies the gadget's
+inverse, with one barrier after both; a gradient item on its own would read
+rows that the next item already writes.  A plan that separates the two must be
+refused.
+"""
+import subprocess
+
+from test_emu_kernels import BUILD, CXX, EMU, FLAGS, drive  # noqa: F401
+
+
+def test_plans_the_kernels_cannot_run_are_refused(drive, tmp_path):  # noqa: F811
+    exe = tmp_path / "plan_checks"
+    objs = [str(BUILD / f"{u}.o") for u in ("kernels_tile_emu", "kernels_stream_emu", "kernels_rtile_emu", "rtile_plan",
+                                            "kernels_batch", "kernels_reduce", "kernels_gemm", "engine", "circuit",
+                                            "emu_rt")]
+    subprocess.run([CXX, *FLAGS, str(EMU / "plan_checks.cpp"), *objs, "-o", str(exe), "-lpthread",
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "ACCEPTED" not in r.stdout, r.stdout + r.stderr
