@@ -134,7 +134,9 @@ __device__ __forceinline__ double grad_apply(cx<R>* phi, cx<R>* lam, uint32_t T,
             });
         } else {
             const unsigned hb = 31u - (unsigned)__builtin_clz(lxy);
-            sweep(T >> 1, std::integral_constant<int, ROWS / 2>{}, std::integral_constant<int, 4>{},
+            // (FP32 tiles have twice the rows: batches of four made the 2^13 kernel
+            // spill 48 bytes per thread, two leave 16 and take 1% less time)
+            sweep(T >> 1, std::integral_constant<int, ROWS / 2>{}, std::integral_constant<int, sizeof(R) == 8 ? 4 : 2>{},
                   [&](uint32_t j, cx<R>* v) {
                       const uint32_t i0 = ins0_32(j, hb), i1 = i0 ^ lxy;
                       v[0] = phi[i0]; v[1] = phi[i1]; v[2] = lam[i0]; v[3] = lam[i1];
@@ -236,10 +238,10 @@ __device__ __forceinline__ void flush_grads(const BatchStage& st, const TileOp* 
 
 // Bound by the phases of each item's LDS sweep: eight waves read, combine and
 // write a tile between two barriers (a 4096-amplitude sweep takes about 2800
-// clocks, its LDS traffic alone 1160).  256 jobs of 10-15 qubits, 50-300 gates:
-// 10.9 ms with angles turned into factors by every thread of every item, phi and
+// clocks, its LDS traffic alone 1160).  256 jobs of 10-15 qubits, 50-300 gates,
+// kernel time: 10.9 ms with angles turned into factors by every thread of every item, phi and
 // lambda swept one after the other and a workgroup reduction per gradient term;
-// 9.2 ms now.
+// 9.1 ms now (a whole run 11.3 and 9.8 ms).
 template <typename R, int TB, int M>
 __global__ __launch_bounds__(TB) void k_batch(const BatchJob* __restrict__ jobs, unsigned numJobs,
                                               const BatchStage* __restrict__ stages,
