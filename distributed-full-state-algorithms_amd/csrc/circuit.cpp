@@ -63,21 +63,47 @@ PauliGroups pauli_groups(const double* coeffs, unsigned T, const unsigned* pauli
     }
     for (size_t g = 0, first = 0; g < h.groups.size(); g++) {
         if ((h.groups[g].mxy ^ h.groups[first].mxy) >> PAULI_CHUNK_BITS) first = g;
-        h.groups[first].run++;
+        if (h.groups[first].run++ == 0) h.runs++;
     }
     return h;
 }
 
+namespace {
+
+// Which form a sum takes (expec: <H>, else H psi).  Groups save loads and leave
+// <H> few partials to add up, but need states that fill the GPU with chunks
+// (2^11 amplitudes), and terms that share: a run of groups reads psi once.
+// Time by groups / term by term:
+//   <H>, 4 or more terms: 1.0-2.6 at 18 qubits and fewer, 0.55-1.07 at 19,
+// 0.27-0.99 at 20, 0.09-0.25 at 24.  One string: 1.04-1.2 if it stays in its
+// chunk, 0.75-0.9 if not (half of the chunks are skipped).
+//   H psi of four times as many terms as runs (Z strings, local Hamiltonians):
+// 0.85-1.4 at 19 qubits, 0.54-1.09 at 20, 0.26-0.97 from 22.  Of other sums, FP64:
+// 0.82-0.92 for 100 terms and more at 20 qubits and 1.0-1.17 for fewer,
+// 0.96 for 64 terms at 21, 0.58-1.06 for 24 and more from 22 and 0.8-1.6 for
+// fewer; FP32: 1.0-1.1 at 20, 0.79-1.07 at 21 but 1.03 for one term, 0.53-1.07
+// from 22.
+bool by_groups(const PauliGroups& h, unsigned n, bool fp64, bool expec) {
+    const unsigned terms = (unsigned)h.signs.size();
+    if (expec) return n >= 20 ? terms >= 2 || h.groups[0].mxy >> PAULI_CHUNK_BITS : terms >= 4;
+    if (4 * h.runs <= terms) return true;
+    return fp64 ? terms >= (n == 20 ? 100u : n == 21 ? 64u : 24u) : n >= 22 || (n == 21 && terms >= 2);
+}
+
+}  // namespace
+
 PauliSumDev push_pauli_sum(ParamRing& ring, const double* coeffs, unsigned T, const unsigned* paulis, unsigned n,
                            int prec, bool expec) {
     PauliSumDev d;
-    if (!pauli_sum_grouped(n, T, prec == FSA_FP64, expec)) {
+    PauliGroups h;
+    const unsigned least = expec ? 19 : 20;      // qubits
+    if (n >= least) h = pauli_groups(coeffs, T, paulis, n);
+    if (T == 0 || n < least || !by_groups(h, n, prec == FSA_FP64, expec)) {
         const std::vector<PauliTermDev> terms = pauli_terms(coeffs, T, paulis, n, false);
         d.terms = static_cast<const PauliTermDev*>(ring.push(terms.data(), T * sizeof(PauliTermDev)));
         d.count = T;
         return d;
     }
-    const PauliGroups h = pauli_groups(coeffs, T, paulis, n);
     // one region: groups, then terms (both multiples of 8 bytes)
     const size_t gb = h.groups.size() * sizeof(PauliGroupDev), tb = h.signs.size() * sizeof(PauliSignDev);
     std::vector<char> blob(gb + tb);

@@ -152,6 +152,7 @@ std::vector<PauliTermDev> pauli_terms(const double* coeffs, unsigned T, const un
 struct PauliGroups {
     std::vector<PauliGroupDev> groups;
     std::vector<PauliSignDev> signs;
+    unsigned runs = 0;          // of groups that agree above the chunk
 };
 PauliGroups pauli_groups(const double* coeffs, unsigned T, const unsigned* paulis, unsigned n);
 // a sum on a statevector in the form for its size (expec: <H>, else H psi), queued to the device

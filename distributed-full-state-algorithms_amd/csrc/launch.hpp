@@ -211,17 +211,6 @@ struct PauliSumDev {
     const PauliTermDev* terms = nullptr;
     unsigned count = 0;
 };
-// Which form a sum takes (expec: <H>, else H psi).  Groups save loads and leave
-// <H> few partials to add up, but need states that fill the GPU with chunks and
-// enough terms to share.  Grouped against term by term, strings of weight 1-4:
-// <H> of 100, 20 and 2 terms in 0.53, 0.63 and 0.94 of the time at 20 qubits FP64,
-// 0.09, 0.25 and 0.62 at 24, but one term 1.2 times as long at 28; H psi of 100 terms 0.89-1.00 at
-// 20 qubits, 0.55-0.67 at 22; FP64 at 22-28, 8 terms 0.65-1.43, 64 terms
-// 0.58-1.03; FP32 48 terms 0.51-0.81 (random strings on all qubits 0.79-0.98,
-// 24 of them 0.84-1.08).
-constexpr bool pauli_sum_grouped(unsigned n, unsigned numTerms, bool fp64, bool expec) {
-    return expec ? n >= 20 && numTerms >= 2 : n >= 22 && numTerms >= (fp64 ? 64u : 48u);
-}
 uint64_t sv_expec_workspace_doubles(unsigned n, const PauliSumDev& h);
 // one adjoint reverse step for a parametrised gadget (kernels_reduce.hip)
 struct AdjointStepDev {
