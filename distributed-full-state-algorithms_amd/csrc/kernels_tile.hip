@@ -508,8 +508,11 @@ unsigned tile_workgroups_per_cu(const void* kern, unsigned tb, size_t lds, unsig
 template <typename R, int TB, int RW>
 auto pick_tile(uint32_t var, bool sw) {
     constexpr int W = sweep_bits<R>();
-    return var == 3 ? k_tile<R, TB, RW, W, 3, false> : var == 2 ? k_tile<R, TB, RW, W, 2, false>
-         : var == 1 ? k_tile<R, TB, RW, W, 1, false>
+    if (var >= 2) {
+        if constexpr (RW >= MFMA_MIN_ROWS) return var == 3 ? k_tile<R, TB, RW, W, 3, false> : k_tile<R, TB, RW, W, 2, false>;
+        fail(FSA_ERR_INTERNAL, "an MFMA pass needs a full tile");
+    }
+    return var == 1 ? k_tile<R, TB, RW, W, 1, false>
          : sw ? k_tile<R, TB, RW, W, 0, true> : k_tile<R, TB, RW, W, 0, false>;
 }
 

@@ -194,6 +194,9 @@ __device__ __forceinline__ uint32_t mat_lds_index(uint32_t r, uint32_t c) {
     return r * (uint32_t)D + (c ^ (r & (uint32_t)(D - 1)));
 }
 
+// amplitudes per thread (T / TB) of the smallest tile that tile_matk_mfma takes
+constexpr int MFMA_MIN_ROWS = 8;
+
 // M holds U as complex entries (mat_lds_index), so a lane gets ur and ui, and xr
 // and xi, in one LDS read each.  A wave owns 16-group column blocks with every
 // row of U: an amplitude is read once per sweep over the k-steps, and since no
@@ -222,10 +225,12 @@ __device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileO
     constexpr bool TWICE = GAUSS && D == 32;
     constexpr int PARTS = GAUSS && !TWICE ? 3 : D >= 16 ? 2 : 1;
     constexpr int WAVES = TB / 64;
-    // column blocks at once (16 to 32 accumulator registers in FP32, 16 to 32 in
-    // FP64); a full tile holds a multiple of NC * WAVES of them
+    // column blocks at once (16 accumulator registers in FP32, 16 to 32 in FP64);
+    // a tile of MFMA_MIN_ROWS amplitudes per thread or more holds a multiple of
+    // NC * WAVES of them
     constexpr int NC = sizeof(R) == 8 ? (D == 8 ? 2 : 1) : 32 / D;
     static_assert(K >= 3 && K <= 5, "three to five targets");
+    static_assert((MFMA_MIN_ROWS * TB >> (K + 4)) % (NC * WAVES) == 0, "a wave's column blocks would leave the tile");
     const uint32_t b0 = 1u << op.p[0], b1 = 1u << op.p[1], b2 = 1u << op.p[2];
     const uint32_t b3 = K > 3 ? 1u << op.p[3] : 0u;
     const uint32_t b4 = K > 4 ? 1u << op.p[4] : 0u;

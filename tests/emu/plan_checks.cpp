@@ -35,6 +35,15 @@ static void plan(const std::vector<HOp>& ops, const std::vector<int>& sign) {
     bb.add_plan(ops, sign, 6, SchedParams{6, 6}, 1, true, first, count);
 }
 
+// an MFMA pass over tiles of 2^m amplitudes
+template <typename R>
+static void mfma_pass(unsigned m) {
+    TileGeom g{};
+    g.m = m;
+    for (unsigned q = 0; q < m; q++) g.tileMask |= 1ULL << q;
+    launch_tile<R>(nullptr, nullptr, m, g, nullptr, 1, nullptr, nullptr, 2u << 2, 0);
+}
+
 int main() {
     const HOp a = gadget(1, 0, 0), b = gadget(2, 0, 1);
     const HOp ga = grad_op(a, 0), gb = grad_op(b, 1), ia = inverse(a), ib = inverse(b);
@@ -43,5 +52,8 @@ int main() {
     refuses("gradient_last", [&] { plan({ia, ga}, {-1, 0}); });
     refuses("gradient_before_another_inverse", [&] { plan({ga, ib, ia}, {0, -1, -1}); });
     refuses("gradient_before_a_forward_gadget", [&] { plan({ga, a}, {0, 1}); });
+    // a wave's column blocks would leave the tile
+    refuses("mfma_pass_on_a_2^11_fp64_tile", [] { mfma_pass<double>(11); });
+    refuses("mfma_pass_on_a_2^11_fp32_tile", [] { mfma_pass<float>(11); });
     return failures ? 1 : 0;
 }

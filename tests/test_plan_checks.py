@@ -3,7 +3,8 @@
 The batch kernel sums a gradient term in the sweep that applies the gadget's
 inverse, with one barrier after both; a gradient item on its own would read
 rows that the next item already writes.  A plan that separates the two must be
-refused.
+refused, and so must an MFMA pass over tiles that do not hold the column blocks
+of every wave.
 """
 import subprocess
 
