@@ -1,0 +1,61 @@
+// The layouts that the adjoint planner gives to register-tile passes, compiled
+// against the CPU stand-in with the planner's source in the same unit: every
+// access of a pass must cover whole 128-byte lines (its stores are streaming
+// ones), so the qubits of a line stay on the low lane bits.  Exit status 0 unless
+// a pass breaks this.
+#include "../../distributed-full-state-algorithms_amd/csrc/circuit.cpp"
+
+#include <cstdio>
+
+static HOp gadget(uint64_t mxy, uint64_t myz, int param) {
+    HOp o;
+    o.kind = OP_PAULI;
+    o.gadget = true;
+    o.mxy = mxy;
+    o.myz = myz;
+    o.theta = 0.3;
+    o.param = param;
+    refresh_angle(o);
+    finish_op(o);
+    return o;
+}
+
+template <typename R>
+static int check(const Circuit& c, unsigned n, bool rev) {
+    Circuit plan = c;
+    const std::vector<Stage>& stages = sweep_stages<R>(plan, n, sizeof(R) == 8 ? FSA_FP64 : FSA_FP32, rev);
+    std::vector<SweepOp> sops;
+    SweepBuilder<R> b(plan, rev, sops);
+    int bad = 0, passes = 0;
+    for (const Stage& st : stages) {
+        if (!st.tiled) continue;
+        for (const SweepPass& p : b.stage(st)) {
+            passes++;
+            bool whole = true;
+            for (unsigned q = 0; (sizeof(cx<R>) << q) < 128; q++)
+                whole = whole && p.geom.lane[q] == q && p.geom.laneOut[q] == q;
+            bad += !whole;
+        }
+    }
+    std::printf("FP%zu rev %d n %u: %d passes, %d not in whole lines\n", 8 * sizeof(R), (int)rev, n, passes, bad);
+    return bad + (passes == 0);
+}
+
+int main() {
+    int bad = 0;
+    for (unsigned n : {12u, 13u, 17u}) {
+        Circuit c;
+        int param = 0;
+        for (unsigned layer = 0; layer < 3; layer++) {
+            for (unsigned q = 0; q + 1 < n; q++) c.ops.push_back(gadget(0, 3ULL << q, param++));
+            // the line's qubits are mixed first, last and most often
+            for (unsigned i = 0; i < n; i++) {
+                const unsigned q = layer == 1 ? n - 1 - i : i;
+                c.ops.push_back(gadget(1ULL << q, layer == 2 ? 1ULL << q : 0, param++));
+            }
+            for (unsigned q = 0; q < 4; q++) c.ops.push_back(gadget(1ULL << q, 1ULL << (n - 1 - q), param++));
+        }
+        for (bool rev : {false, true}) bad += check<double>(c, n, rev) + check<float>(c, n, rev);
+    }
+    return bad ? 1 : 0;
+}
