@@ -220,8 +220,10 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_step(cx<R>* __restrict__ phi,
 // U^dag factors, looked up by the amplitude's parity pattern (bit g = parity
 // of gadget g) in a table each block builds in LDS.  Each accumulator then
 // takes the same two-level reduction as k_adjoint_step: block sums here (one
-// row per workgroup in the gadget's slot), then k_grad_sums.
-template <typename R, bool WIDE>
+// row per workgroup in the gadget's slot), then k_grad_sums.  This kernel and
+// the two below serve the states too small for register-tile passes
+// (sweep_min_qubits), where a launch is what counts.
+template <typename R>
 __global__ __launch_bounds__(BLOCK) void k_adjoint_diag(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
                                                         uint64_t num, AdjointDiagDev st, double* __restrict__ rows,
                                                         uint64_t stride) {
@@ -237,24 +239,23 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_diag(cx<R>* __restrict__ phi,
     double vr[ADJ_DIAG_MAX], vi[ADJ_DIAG_MAX];
 #pragma unroll
     for (unsigned g = 0; g < ADJ_DIAG_MAX; g++) { vr[g] = 0; vi[g] = 0; }
-    for (uint64_t k = adjoint_block<R>() * BLOCK + threadIdx.x; k < num; k += (uint64_t)gridDim.x * BLOCK) {
-        const cx<R> p = adj_ld<R, true>(phi + k), l = adj_ld<R, true>(lam + k);
+    for (uint64_t k = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; k < num; k += (uint64_t)gridDim.x * BLOCK) {
+        const cx<R> p = phi[k], l = lam[k];
         const double wr = (double)l.x * (double)p.x + (double)l.y * (double)p.y;
         const double wi = (double)l.x * (double)p.y - (double)l.y * (double)p.x;
         unsigned pat = 0;
 #pragma unroll
         for (unsigned g = 0; g < ADJ_DIAG_MAX; g++) {
             if (g < cnt) {
-                // WIDE: states of more than 32 qubits (64-bit parities)
-                const unsigned odd = WIDE ? par64(k & st.myz[g]) : par32((uint32_t)k & (uint32_t)st.myz[g]);
+                const unsigned odd = par32((uint32_t)k & (uint32_t)st.myz[g]);
                 pat |= odd << g;
                 vr[g] += odd ? -wr : wr;
                 vi[g] += odd ? -wi : wi;
             }
         }
         const cx<R> f = tab[pat];
-        adj_st<R, true>(phi + k, cmul(p, f));
-        adj_st<R, true>(lam + k, cmul(l, f));
+        phi[k] = cmul(p, f);
+        lam[k] = cmul(l, f);
     }
 #pragma unroll
     for (unsigned g = 0; g < ADJ_DIAG_MAX; g++) {
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_diag(cx<R>* __restrict__ phi,
 // values (conj(lambda_j) s(j') phi_j' over its pairs j' = j ^ bit, as in
 // k_adjoint_step), then applies every gadget's U^dag to its pairs and writes
 // the group back.  Reduction as in k_adjoint_diag.
-template <typename R, int G, bool NT>
+template <typename R, int G>
 __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
                                                         uint64_t numGroups, AdjointQubitRunDev st,
                                                         double* __restrict__ rows, uint64_t stride) {
@@ -292,13 +293,13 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun(cx<R>* __restrict__ phi,
 #pragma unroll
         for (int g = 0; g < G; g++) if ((e >> g) & 1u) off[e] |= 1ULL << st.q[g];
     }
-    for (uint64_t t = adjoint_block<R>() * BLOCK + threadIdx.x; t < numGroups; t += (uint64_t)gridDim.x * BLOCK) {
+    for (uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; t < numGroups; t += (uint64_t)gridDim.x * BLOCK) {
         uint64_t x = t;
 #pragma unroll
         for (int i = 0; i < G; i++) x = ins0(x, st.sorted[i]);
         cx<R> p[E], l[E];
 #pragma unroll
-        for (unsigned e = 0; e < E; e++) { p[e] = adj_ld<R, NT>(phi + (x | off[e])); l[e] = adj_ld<R, NT>(lam + (x | off[e])); }
+        for (unsigned e = 0; e < E; e++) { p[e] = phi[x | off[e]]; l[e] = lam[x | off[e]]; }
 #pragma unroll
         for (int g = 0; g < G; g++) {
             // s(j) = -1 where the gadget is Y and j has its qubit set (the pair's second element)
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun(cx<R>* __restrict__ phi,
             }
         }
 #pragma unroll
-        for (unsigned e = 0; e < E; e++) { adj_st<R, NT>(phi + (x | off[e]), p[e]); adj_st<R, NT>(lam + (x | off[e]), l[e]); }
+        for (unsigned e = 0; e < E; e++) { phi[x | off[e]] = p[e]; lam[x | off[e]] = l[e]; }
     }
 #pragma unroll
     for (int g = 0; g < G; g++) {
@@ -358,7 +359,7 @@ __device__ __forceinline__ cx<R> shfl_xor_cx(cx<R> v, int m) {
 // DG: the diagonal run that follows in the sweep (dg, 1..ADJ_DIAG_MAX gadgets)
 // is applied in the same pass, after the run, as k_adjoint_diag does it: its
 // terms from the updated amplitudes, then its factors from an LDS table.
-template <typename R, int G, bool DG, bool WIDE>
+template <typename R, int G, bool DG>
 __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
                                                              uint64_t num, AdjointQubitRunDev st, AdjointDiagDev dg,
                                                              double* __restrict__ rows, uint64_t stride) {
@@ -380,8 +381,8 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
 #pragma unroll
     for (int g = 0; g < DM; g++) { dr[g] = 0; di[g] = 0; }
     // num is a multiple of 64 and so is the stride: a wave's lanes stay together
-    for (uint64_t j = adjoint_block<R>() * BLOCK + threadIdx.x; j < num; j += (uint64_t)gridDim.x * BLOCK) {
-        cx<R> p = adj_ld<R, true>(phi + j), l = adj_ld<R, true>(lam + j);
+    for (uint64_t j = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; j < num; j += (uint64_t)gridDim.x * BLOCK) {
+        cx<R> p = phi[j], l = lam[j];
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const cx<R> pp = shfl_xor_cx(p, 1 << st.q[g]);
@@ -408,8 +409,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
 #pragma unroll
             for (unsigned g = 0; g < ADJ_DIAG_MAX; g++) {
                 if (g < cnt) {
-                    // WIDE: states of more than 32 qubits (64-bit parities)
-                    const unsigned odd = WIDE ? par64(j & dg.myz[g]) : par32((uint32_t)j & (uint32_t)dg.myz[g]);
+                    const unsigned odd = par32((uint32_t)j & (uint32_t)dg.myz[g]);
                     pat |= odd << g;
                     dr[g] += odd ? -wr : wr;
                     di[g] += odd ? -wi : wi;
@@ -419,8 +419,8 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
             p = cmul(p, fd);
             l = cmul(l, fd);
         }
-        adj_st<R, true>(phi + j, p);
-        adj_st<R, true>(lam + j, l);
+        phi[j] = p;
+        lam[j] = l;
     }
 #pragma unroll
     for (int g = 0; g < G; g++) {
@@ -840,10 +840,10 @@ unsigned launch_adjoint_step(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq,
 template <typename R>
 unsigned launch_adjoint_diag(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const AdjointDiagDev& st,
                              double* rows, uint64_t stride) {
+    if (nq > 32) fail(FSA_ERR_INTERNAL, "adjoint run of diagonal gadgets on more than 32 qubits");
     const uint64_t num = 1ULL << nq;
     const unsigned nb = red_blocks(num);
-    auto* kern = nq > 32 ? k_adjoint_diag<R, true> : k_adjoint_diag<R, false>;
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(BLOCK), 0, s, phi, lam, num, st, rows, stride);
+    hipLaunchKernelGGL(k_adjoint_diag<R>, dim3(nb), dim3(BLOCK), 0, s, phi, lam, num, st, rows, stride);
     return nb;
 }
 
@@ -851,7 +851,7 @@ template <typename R>
 unsigned launch_adjoint_qrun(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq, const AdjointQubitRunDev& st,
                              double* rows, uint64_t stride, const AdjointDiagDev* tail) {
     const unsigned G = st.count;
-    if (G < 2 || G > ADJ_QRUN_MAX || nq < G) fail(FSA_ERR_INTERNAL, "adjoint qubit run of unsupported length");
+    if (G < 2 || G > ADJ_QRUN_MAX || nq < G || nq > 32) fail(FSA_ERR_INTERNAL, "adjoint qubit run of unsupported length");
     const uint64_t numGroups = 1ULL << (nq - G);
     uint64_t bits = 0;
     for (unsigned g = 0; g < G; g++) bits |= 1ULL << st.q[g];
@@ -862,30 +862,24 @@ unsigned launch_adjoint_qrun(hipStream_t s, cx<R>* phi, cx<R>* lam, unsigned nq,
         AdjointDiagDev dg;
         std::memset(&dg, 0, sizeof(dg));
         if (tail) dg = *tail;
-#define FSA_QL(GV, DGV, WV)                                                                                       \
-        hipLaunchKernelGGL((k_adjoint_qrun_lane<R, GV, DGV, WV>), dim3(nbl), dim3(BLOCK), 0, s, phi, lam, num, st, \
-                           dg, rows, stride)
-        const bool wide = nq > 32;
+#define FSA_QL(GV, DGV)                                                                                          \
+        hipLaunchKernelGGL((k_adjoint_qrun_lane<R, GV, DGV>), dim3(nbl), dim3(BLOCK), 0, s, phi, lam, num, st, dg, \
+                           rows, stride)
         if (G == 2) {
-            if (!tail) FSA_QL(2, false, false);
-            else if (wide) FSA_QL(2, true, true);
-            else FSA_QL(2, true, false);
+            if (tail) FSA_QL(2, true);
+            else FSA_QL(2, false);
         } else {
-            if (!tail) FSA_QL(3, false, false);
-            else if (wide) FSA_QL(3, true, true);
-            else FSA_QL(3, true, false);
+            if (tail) FSA_QL(3, true);
+            else FSA_QL(3, false);
         }
 #undef FSA_QL
         return nbl;
     }
     if (tail) fail(FSA_ERR_INTERNAL, "a diagonal tail needs a qubit run below qubit 6");
     const unsigned nb = red_blocks(numGroups);
-    const bool nt = (bits & (128 / sizeof(cx<R>) - 1)) == 0;
-#define FSA_QR(GV)                                                                                                \
-    if (G == GV) {                                                                                                \
-        auto* kern = nt ? k_adjoint_qrun<R, GV, true> : k_adjoint_qrun<R, GV, false>;                             \
-        hipLaunchKernelGGL(kern, dim3(nb), dim3(BLOCK), 0, s, phi, lam, numGroups, st, rows, stride);             \
-    }
+#define FSA_QR(GV)                                                                                                 \
+    if (G == GV)                                                                                                   \
+        hipLaunchKernelGGL((k_adjoint_qrun<R, GV>), dim3(nb), dim3(BLOCK), 0, s, phi, lam, numGroups, st, rows, stride);
     FSA_QR(2) FSA_QR(3)
 #undef FSA_QR
     return nb;
