@@ -158,13 +158,12 @@ struct SweepOp {
 constexpr unsigned SWEEP_LANE_BITS = 6;
 // register bits: 64 VGPRs of amplitudes (rev: of phi and lambda together)
 template <typename R> constexpr unsigned sweep_reg_bits(bool rev) { return (sizeof(R) == 8 ? 4u : 5u) - (rev ? 1u : 0u); }
-// Smallest states that the passes take.  Smaller ones give a pass one or two
-// waves, which run its ops one after another, and the run kernels' launches of
-// a few us each are no slower.  20 layers of ZZ and X gadgets, ms per gradient,
-// passes against run kernels: 1.05 / 1.22 at 10 qubits FP64; in FP32 1.42 / 1.70 at
-// 12, while at 10 and 11 an earlier form of the passes took 1.33 / 1.20 and
-// 1.49 / 1.39.
-template <typename R> constexpr unsigned sweep_min_qubits() { return sizeof(R) == 8 ? 10u : 12u; }
+// Smallest states that the passes take: those that fill one forward tile.  Passes
+// against run kernels, us per gradient of 20 layers (2 layers): ZZ and X gadgets
+// 687 / 928 (138 / 159) at 10 qubits FP64, 921 / 1091 (177 / 189) at 11 qubits
+// FP32; Y and Z gadgets with CNOTs 1037 / 1901 and 1497 / 2192; random strings of
+// weight 1-4 643 / 768 (122 / 149) and 843 / 961 (185 / 184).
+template <typename R> constexpr unsigned sweep_min_qubits() { return sizeof(R) == 8 ? 10u : 11u; }
 constexpr unsigned SWEEP_MAX_GRADS = 46;     // gradient terms of a pass: two per 2 KiB row of LDS
 struct SweepGeom {
     uint64_t tileMask;

@@ -43,7 +43,7 @@ static int check(const Circuit& c, unsigned n, bool rev) {
 
 int main() {
     int bad = 0;
-    for (unsigned n : {12u, 13u, 17u}) {
+    for (unsigned n : {11u, 12u, 13u, 17u}) {
         Circuit c;
         int param = 0;
         for (unsigned layer = 0; layer < 3; layer++) {
