@@ -205,9 +205,14 @@ constexpr int MFMA_MIN_ROWS = 8;
 //   FP32, 4 or 5 targets: Yr and Yi apart, four products: 1 + RB LDS reads feed
 // 4 RB matrix operations.
 //   FP64, 4 targets: Gauss's three products P1 = Ur Xr, P2 = Ui Xi and
-// P3 = (Ur + Ui)(Xr + Xi) in one sweep; Yr = P1 - P2, Yi = P3 - (P1 + P2).
+// P3 = (Ur + Ui)(Xr + Xi) in one sweep; Yr = P1 - P2, Yi = P3 - (P1 + P2).  P3, the
+// largest, is summed in two halves, the even and the odd k-steps: 30 gates on 14
+// qubits end 1.017e-15 off, with one sum 1.100e-15 (with P3 added to -(P1 + P2) in
+// a second sweep 1.076e-15, and 60 gates on 25 qubits take 6.56 instead of 6.09 ms).
 //   FP64, 5 targets: P3 in a second sweep, added to -(P1 + P2): the 48
 // accumulator registers of one sweep over both row blocks make the kernel spill.
+//   FP64 tiles of 2^13 on 1024 threads: four products (60 gates on 15 qubits
+// 1.12e-15 off; with three 1.22e-15).
 //   3 targets: the 16 rows of one operation are Yr and Yi of the 8 outputs.
 // Bound by the matrix unit, whose operations (64 cycles in FP64, 32 in FP32)
 // hide the reads once two workgroups share a CU.  Tasks of one 16-row block
@@ -221,9 +226,9 @@ __device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileO
     typedef typename MfmaAcc<R>::T acc_t;
     constexpr int D = 1 << K;
     constexpr int RB = D >= 16 ? D / 16 : 1;              // 16-row blocks of U
-    constexpr bool GAUSS = D >= 16 && sizeof(R) == 8;
+    constexpr bool GAUSS = D >= 16 && sizeof(R) == 8 && TB == 512;
     constexpr bool TWICE = GAUSS && D == 32;
-    constexpr int PARTS = GAUSS && !TWICE ? 3 : D >= 16 ? 2 : 1;
+    constexpr int PARTS = GAUSS && !TWICE ? 4 : D >= 16 ? 2 : 1;
     constexpr int WAVES = TB / 64;
     // column blocks at once (16 accumulator registers in FP32, 16 to 32 in FP64);
     // a tile of MFMA_MIN_ROWS amplitudes per thread or more holds a multiple of
@@ -252,31 +257,35 @@ __device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileO
 #pragma unroll
                 for (int h = 0; h < PARTS; h++) acc[c][b][h] = acc_t{0, 0, 0, 0};
         }
+        constexpr int STEPS = GAUSS && !TWICE ? 2 : 1;    // per round: even and odd ones
 #pragma unroll 1
-        for (uint32_t ks = 0; ks < (uint32_t)(D / 4); ks++) {
-            const uint32_t col = ks * 4 + lk;             // column of U = row of X
-            const uint32_t off = mat_offset<K>(col, b0, b1, b2, b3, b4);
-            cx<R> x[NC];
+        for (uint32_t ks = 0; ks < (uint32_t)(D / 4); ks += STEPS) {
 #pragma unroll
-            for (int c = 0; c < NC; c++) x[c] = s[gb[c] | off];
+            for (int half = 0; half < STEPS; half++) {
+                const uint32_t col = (ks + half) * 4 + lk;    // column of U = row of X
+                const uint32_t off = mat_offset<K>(col, b0, b1, b2, b3, b4);
+                cx<R> x[NC];
 #pragma unroll
-            for (int b = 0; b < RB; b++) {
-                const cx<R> u = M[mat_lds_index<D>(((uint32_t)b * 16 + lr) & (D - 1), col)];
-                // what multiplies xr and xi in this lane's row of the first accumulator
-                R ar = u.x, ai = -u.y;
-                if (PARTS == 1 && lr >= (uint32_t)D) { ar = u.y; ai = u.x; }
+                for (int c = 0; c < NC; c++) x[c] = s[gb[c] | off];
 #pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    acc_t* y = acc[c][b];
-                    y[0] = MfmaAcc<R>::step(ar, x[c].x, y[0]);
-                    if constexpr (GAUSS) {
-                        y[1] = MfmaAcc<R>::step(u.y, x[c].y, y[1]);
-                        if constexpr (!TWICE) y[2] = MfmaAcc<R>::step(u.x + u.y, x[c].x + x[c].y, y[2]);
-                    } else {
-                        y[0] = MfmaAcc<R>::step(ai, x[c].y, y[0]);
-                        if constexpr (PARTS == 2) {
-                            y[1] = MfmaAcc<R>::step(u.y, x[c].x, y[1]);
-                            y[1] = MfmaAcc<R>::step(u.x, x[c].y, y[1]);
+                for (int b = 0; b < RB; b++) {
+                    const cx<R> u = M[mat_lds_index<D>(((uint32_t)b * 16 + lr) & (D - 1), col)];
+                    // what multiplies xr and xi in this lane's row of the first accumulator
+                    R ar = u.x, ai = -u.y;
+                    if (PARTS == 1 && lr >= (uint32_t)D) { ar = u.y; ai = u.x; }
+#pragma unroll
+                    for (int c = 0; c < NC; c++) {
+                        acc_t* y = acc[c][b];
+                        y[0] = MfmaAcc<R>::step(ar, x[c].x, y[0]);
+                        if constexpr (GAUSS) {
+                            y[1] = MfmaAcc<R>::step(u.y, x[c].y, y[1]);
+                            if constexpr (!TWICE) y[2 + half] = MfmaAcc<R>::step(u.x + u.y, x[c].x + x[c].y, y[2 + half]);
+                        } else {
+                            y[0] = MfmaAcc<R>::step(ai, x[c].y, y[0]);
+                            if constexpr (PARTS == 2) {
+                                y[1] = MfmaAcc<R>::step(u.y, x[c].x, y[1]);
+                                y[1] = MfmaAcc<R>::step(u.x, x[c].y, y[1]);
+                            }
                         }
                     }
                 }
@@ -310,7 +319,7 @@ __device__ __forceinline__ void tile_matk_mfma(cx<R>* s, uint32_t T, const TileO
                     const uint32_t row = (uint32_t)b * 16 + (sizeof(R) == 8 ? 4u * (uint32_t)j + lk : lk * 4u + (uint32_t)j);
                     cx<R>* dst = &s[gb[c] | mat_offset<K>(row & (D - 1), b0, b1, b2, b3, b4)];
                     const acc_t* y = acc[c][b];
-                    if constexpr (PARTS == 3) *dst = mk<R>(y[0][j] - y[1][j], y[2][j] - (y[0][j] + y[1][j]));
+                    if constexpr (PARTS == 4) *dst = mk<R>(y[0][j] - y[1][j], (y[2][j] - (y[0][j] + y[1][j])) + y[3][j]);
                     else if constexpr (PARTS == 2) *dst = mk<R>(y[0][j], y[1][j]);
                     else reinterpret_cast<R*>(dst)[row < (uint32_t)D ? 0 : 1] = y[0][j];
                 }
