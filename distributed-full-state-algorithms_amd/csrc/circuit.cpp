@@ -350,8 +350,8 @@ private:
         }
         sops_.push_back(t);
     }
-    // -tan(a / 2) of the rotation with cosine t.c >= 0 and sine t.g
-    static double shear_t(const SweepOp& t) { return -t.g / (1.0 + t.c); }
+    // turn()'s c for the rotation with cosine t.c >= 0 and sine t.g: -tan(a / 2), or t.c itself
+    double turn_c(const SweepOp& t) const { return sizeof(R) == 8 || rev_ ? -t.g / (1.0 + t.c) : t.c; }
 
     // diagonal ops commute: those with the same slot signs go together
     void flush_run() {
@@ -365,7 +365,7 @@ private:
             const uint32_t one = SWEEP_GROUP_FIRST | SWEEP_GROUP_LAST;
             if ((ts[i].first.flags & one) == one) {
                 ts[i].first.code += SWEEP_DIAG_ONE - SWEEP_DIAG;
-                ts[i].first.c = shear_t(ts[i].first);
+                ts[i].first.c = turn_c(ts[i].first);
             }
             emit(ts[i].first, ts[i].second);
         }
@@ -420,7 +420,7 @@ private:
         if (y) t.g = -sn;
         if (onReg) {
             t.code = SWEEP_REG + 4u * (uint32_t)rb;
-            t.c = shear_t(t);
+            t.c = turn_c(t);
         } else {
             t.code = SWEEP_LANE + 4u * (uint32_t)lane_bit(q);
             if (y) t.lz |= SWEEP_CONST_SIGN;         // the factor is the partner lane's

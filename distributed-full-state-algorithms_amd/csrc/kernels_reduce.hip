@@ -529,7 +529,7 @@ __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi
                 }
                 w = sweep::flip(dsum, sb);
                 if (hdr.code >= SWEEP_DIAG_ONE) {
-                    const R T = (R)sweep::flip(hdr.c, sb);
+                    const R T = (R)(sweep::sweep_shears<R, REV>() ? sweep::flip(hdr.c, sb) : hdr.c);
                     if (ss) sweep::op_diag<R, S, REV, true, true>(v, T, (R)g, hdr.sw);
                     else sweep::op_diag<R, S, REV, true, false>(v, T, (R)g, hdr.sw);
                 } else {
