@@ -173,7 +173,10 @@ struct BatchStage {
     uint32_t pad;
 };
 
-// gradient items per stage: their per-wave sums share the LDS left by the tiles
+// Gradient items per stage: their per-wave sums share the LDS left by the tiles.
+// Stages of more are run in parts, each of which streams phi and lambda once more,
+// but a part is bound by its 96 sweeps, not by that: 64 circuits of 15 qubits with
+// 120 gadgets to a stage take 6.43 ms, and 6.41 with 224 items per stage.
 constexpr uint32_t BATCH_STAGE_GRADS = 96;
 
 struct BatchJob {

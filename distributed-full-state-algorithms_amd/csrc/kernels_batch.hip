@@ -134,9 +134,9 @@ __device__ __forceinline__ double grad_apply(cx<R>* phi, cx<R>* lam, uint32_t T,
             });
         } else {
             const unsigned hb = 31u - (unsigned)__builtin_clz(lxy);
-            // (FP32 tiles have twice the rows: batches of four made the 2^13 kernel
-            // spill 48 bytes per thread, two leave 16 and take 1% less time)
-            sweep(T >> 1, std::integral_constant<int, ROWS / 2>{}, std::integral_constant<int, sizeof(R) == 8 ? 4 : 2>{},
+            // (FP32 tiles of 2^13: batches of four made that kernel spill 48 bytes per
+            // thread, two leave 16 and take 1% less time; with two, the 2^12 kernel spills)
+            sweep(T >> 1, std::integral_constant<int, ROWS / 2>{}, std::integral_constant<int, sizeof(R) == 4 && ROWS >= 16 ? 2 : 4>{},
                   [&](uint32_t j, cx<R>* v) {
                       const uint32_t i0 = ins0_32(j, hb), i1 = i0 ^ lxy;
                       v[0] = phi[i0]; v[1] = phi[i1]; v[2] = lam[i0]; v[3] = lam[i1];
@@ -202,9 +202,11 @@ __device__ __forceinline__ void run_items(cx<R>* phi, uint32_t T, uint64_t base,
     for (uint32_t i = i0; i < i0 + ni; i++) {
         TileOp op = items[i];
         if (REV && op.kind == OP_GRAD) {
-            TileOp inv = items[++i];        // the planner puts the gadget's inverse next to it
+            TileOp inv = items[i + 1];      // the planner puts the gadget's inverse next to it
             bind_param(inv, cs);
-            const double v = bwave_sum(grad_apply<R, TB, ROWS>(phi, lam, T, base, op, inv));
+            double v = grad_apply<R, TB, ROWS>(phi, lam, T, base, op, inv);
+            i++;
+            v = bwave_sum(v);
             if ((threadIdx.x & 63u) == 0) {
                 double* r = gacc + (threadIdx.x >> 6) * BATCH_STAGE_GRADS + op.p[0];
                 *r = firstTile ? v : *r + v;
