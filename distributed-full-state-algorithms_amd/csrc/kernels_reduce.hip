@@ -456,13 +456,14 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_qrun_lane(cx<R>* __restrict__
 // second's, so one exchange folds both and a row of 256 doubles serves two.
 // Three workgroups of four waves per CU (VGPRs and LDS): more waves hide more
 // of the loads and of the scalar work between ops.
-// 20 layers of ZZ and X gadgets, 24 qubits FP64: 35 reverse passes of 315 us (210 us of
+// 20 layers of ZZ and X gadgets, 24 qubits FP64: 35 reverse passes of 310 us (210 us of
 // them the bare loads and stores, against 160 run passes of 197 us and 40
-// diagonal passes of 193 us), 26 forward passes of 147 us (against 19 LDS tile
-// passes of 602 us); 23 qubits FP32: 33 of 135 us and 23 of 46 us.  Bound by
-// vector instructions.  Exchanges through LDS instead of DPP moves and
-// layout changes took 375 us a reverse pass, diagonal gadgets one by one and
-// rotations without shears 336 us.
+// diagonal passes of 193 us), 26 forward passes of 140 us (against 19 LDS tile
+// passes of 602 us); FP32: 36 of 237 us and 23 of 89 us.  Bound by vector
+// instructions (the vector unit is busy 62% and 54% of the time in FP64, 77% and
+// 87% in FP32).  Exchanges through LDS instead of DPP moves and layout changes
+// took 375 us a reverse pass, diagonal gadgets one by one and rotations without
+// shears 336 us.
 template <typename R, int G, bool REV>
 __global__ __launch_bounds__(BLOCK, 3) void k_wave_sweep(cx<R>* __restrict__ phi, cx<R>* __restrict__ lam,
                                                          uint64_t numTiles, SweepGeom geom,

@@ -132,7 +132,8 @@ template <typename R> constexpr int sweep_bits() { return sizeof(R) == 8 ? 2 : 4
 // (matrices: where slot i's controls are set).  Bit 6 of lz is a constant sign.
 enum SweepCode : uint32_t {
     SWEEP_DIAG = 0,      // (+ ss) diagonal gadget of a group: v' = v (c + i g s), s = +-1 by parity
-    SWEEP_DIAG_ONE = 2,  // (+ ss) a group of one: the same with c = -tan(a/2), g = sin a (shears)
+    SWEEP_DIAG_ONE = 2,  // (+ ss) a group of one: the same with c = -tan(a/2), g = sin a (shears;
+                         // FP32 forward passes: c = cos a)
     SWEEP_LANE = 4,      // (+ 4 b + 2 imag + ss) Pauli string with its X/Y qubit on lane bit b < 4:
                          // v' = c v + (imag ? i g : g) s w, w the partner
     SWEEP_REG = 20,      // (+ 4 B + 2 imag + ss) ... on register bit B, c and g as in SWEEP_DIAG_ONE
